@@ -159,8 +159,13 @@ __global__ void __launch_bounds__(512, 2) xs_kernel(const LowrankGemmArgs g) {
   // ---- resident W: fragment [j][s] holds W row fw + 8 (r >> 2) + 4 j + (r & 3), r = lane & 15,
   // k = 128 grp + 8 s. MFMA output element e of column block j in lane l is then column
   // fw + 8 (l >> 4) + 4 j + e: the lane's 8 columns are contiguous.
+  // A row-major W comes through LDS: the wave loads WROWS of its rows at a time as whole 1 KiB rows (full lines) into
+  // its own part of the ring, at the x rows' 1040-byte skew, and reads the fragments as it will read x. Read straight
+  // from memory a fragment is 64 pieces of 16 bytes in 64 different lines, 32 times per wave: that prologue took 6-7
+  // of the 12-15 us a launch costs before its first block (2048 rows: c_fc 19.5 -> 12.2 us, q|k 17.7 -> 10.4, v 13.6
+  // -> 8.1, c_proj 13.2 -> 7.5).
   bf16x8 wr[2][KS];
-  {
+  if (g.w_tiled) {
     const int r = lane & 15;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -168,13 +173,38 @@ __global__ void __launch_bounds__(512, 2) xs_kernel(const LowrankGemmArgs g) {
       const long n = QK ? qk_col(nslice, wave, lcol) : fw + lcol;
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
-        const long k = 128 * grp + 8 * s;  // 8 columns of one 16-byte chunk, in either layout
-        wr[j][s] = *reinterpret_cast<const bf16x8*>(g.W + (g.w_tiled ? wtile_offset(n, k, KD) : n * g.ldw + k));
+        const long k = 128 * grp + 8 * s;  // 8 columns of one 16-byte chunk
+        wr[j][s] = *reinterpret_cast<const bf16x8*>(g.W + wtile_offset(n, k, KD));
       }
     }
+    // the fragments have landed before any LDS-bound load is issued, so no wait below covers them
+    wait_vm_lgkm0<0>();
+  } else {
+    constexpr int WROWS = NB * R / NW >= 16 ? 16 : 8;  // rows per wave that the ring holds at once
+    char* const wl = smem + wave * (WROWS * XROW);
+    const int r = lane & 15;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int h = 0; h < 16 / WROWS; ++h) {
+#pragma unroll
+        for (int q = 0; q < WROWS / 4; ++q) {
+          // rows r = WROWS h + 4 q .. + 3 of the fragment: four consecutive rows of W
+          const int lcol = 8 * ((WROWS * h >> 2) + q) + 4 * j;
+          const bf16* wb = g.W + (long)(QK ? qk_col(nslice, wave, lcol) : fw + lcol) * g.ldw;
+          dma_x4_s4<XROW>(wb, wb + g.ldw, wb + 2 * g.ldw, wb + 3 * g.ldw, 16u * lane, wl + 4 * q * XROW);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");  // the wave's own rows: no barrier
+        if (WROWS == 16 || (r >> 3) == h) {
+#pragma unroll
+          for (int s = 0; s < KS; ++s)
+            wr[j][s] = *reinterpret_cast<const bf16x8*>(wl + (r % WROWS) * XROW + 256 * grp + 16 * s);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");  // read before the next rows (or x) overwrite them
+      }
+    // every wave has read its W rows before another wave's x rows land on them
+    __builtin_amdgcn_s_barrier();
   }
-  // the resident fragments have landed before any LDS-bound load is issued, so no wait below covers them
-  wait_vm_lgkm0<0>();
 
   auto blk_of = [&](int k) { return lo + stream + k * streams; };
 
