@@ -9,7 +9,8 @@
 // Layouts (row-major, K contiguous): A [M, K] bf16 with M = members x T rows (member p owns rows
 // p*T .. p*T+T-1); W [N, K] bf16 in the reference's nn.Linear orientation [out, in].
 //
-// Schedule. The kernel is persistent: one workgroup per CU walks a list of BM x BN output tiles.
+// Schedule. The kernel is persistent: one workgroup per CU (two or four with the smaller tiles that a launch of few
+// rows takes, see pick_tile) walks a list of BM x BN output tiles.
 // Hardware deals workgroups round-robin over the 8 XCDs, so workgroup b serves XCD b % 8; each XCD
 // owns one contiguous range of tiles (N fastest), which keeps the x rows shared by neighbouring
 // tiles in that XCD's L2.
@@ -35,7 +36,6 @@
 // first STAGES stages, then runs this tile's epilogue from LDS-staged vectors; the stores drain
 // while the next tile's operands land.
 #include <algorithm>
-
 #include <type_traits>
 
 #include "common.h"
@@ -58,7 +58,8 @@ struct Cfg {
   static constexpr int LB = BN / ROWS_PER_DMA / NW;  // (W tile)
   static constexpr int L = LA + LB;
   static constexpr int STAGE = (BM + BN) * BK;   // bf16 elements per LDS stage
-  static constexpr int UGROUPS = NTH / BM;       // threads summing one row's x.b partials
+  // threads summing one row's x.b partials: two halves at most, so that every configuration adds them in one order
+  static constexpr int UGROUPS = NTH / BM < 2 ? NTH / BM : 2;
   static_assert(BK == 32 || BK == 64, "BK must be 32 or 64");
   static_assert(WM % 16 == 0 && WN % 16 == 0 && FN % 2 == 0, "wave tile must be a multiple of 16 x 32");
   static_assert(LA * ROWS_PER_DMA * NW == BM && LB * ROWS_PER_DMA * NW == BN, "DMA must tile evenly");
@@ -233,11 +234,13 @@ lowrank_gemm_kernel(const LowrankGemmArgs g) {
     if (F16 && tid < BN / 4) pre_sc = *reinterpret_cast<const float4*>(g.col_scale + n0 + 4 * tid);
     if (tid == 0) pre_sign = pfirst == plast ? g.sign[pfirst] : 0.f;
     const int row = min(m0 + tid % BM, g.M - 1), grp = tid / BM;
-    const int q0 = grp * g.u_parts / C::UGROUPS, q1 = (grp + 1) * g.u_parts / C::UGROUPS;
-    const float* up = g.u + (long)row * g.u_ld + (long)seg * g.u_parts * g.u_qstride;
-    float u = 0.f;
-    for (int q = q0; q < q1; ++q) u += up[q * g.u_qstride];
-    pre_u = u;
+    if (grp < C::UGROUPS) {
+      const int q0 = grp * g.u_parts / C::UGROUPS, q1 = (grp + 1) * g.u_parts / C::UGROUPS;
+      const float* up = g.u + (long)row * g.u_ld + (long)seg * g.u_parts * g.u_qstride;
+      float u = 0.f;
+      for (int q = q0; q < q1; ++q) u += up[q * g.u_qstride];
+      pre_u = u;
+    }
     // the head: the tile's target tokens, so that its epilogue makes no global load (a load there, issued after the
     // next tile's stage loads, would wait for all of them: vector memory operations complete in issue order)
     // (a token id past the int range, like a negative one, matches no column)
@@ -261,7 +264,7 @@ lowrank_gemm_kernel(const LowrankGemmArgs g) {
       if (tid < BN / 4) *reinterpret_cast<float4*>(&ep_a[4 * tid]) = pre_ab;
     }
     if (tid == 0) ep_sign = pre_sign;
-    ep_u[tid / BM][tid % BM] = pre_u;
+    if (tid < C::UGROUPS * BM) ep_u[tid / BM][tid % BM] = pre_u;
     if (CE && tid < BM) ep_t[tid] = pre_t;
   };
 
@@ -335,7 +338,7 @@ lowrank_gemm_kernel(const LowrankGemmArgs g) {
   // does not fit an XCD's L2), which walks groups of CE_GROUP row blocks per column tile so each W column tile
   // is read once per group rather than once per row block (measured: config 3 15.4 -> 14.7 ms; groups of 4:
   // 14.8, 16: 15.3, 32: 17.4).
-  constexpr int CE_GROUP = 8;
+  constexpr int CE_GROUP = 8 * 256 / BM;
   auto tile_mn = [&](int t, int which) {
     if (CE) {
       const int span = CE_GROUP * tiles_n, grp = t / span, rem = t % span;
@@ -576,30 +579,11 @@ lowrank_gemm_kernel(const LowrankGemmArgs g) {
   }
 }
 
-// Tile configurations: <BM, BN, BK, STAGES, WGM, WGN>.
-#ifndef NOISE_GEMM_CFG
-#define NOISE_GEMM_CFG 0
-#endif
-// <BM, BN, BK, STAGES, WGM, WGN, OCC>: OCC workgroups of WGM x WGN waves share a CU.
-#if NOISE_GEMM_CFG == 0
+// Tile configurations <BM, BN, BK, STAGES, WGM, WGN, OCC>: OCC workgroups of WGM x WGN waves share a CU.
 #define CFG_BIG 256, 256, 32, 4, 2, 4, 1
-#define CFG_SMALL 256, 128, 32, 4, 4, 2, 1
-#elif NOISE_GEMM_CFG == 1
-#define CFG_BIG 256, 256, 64, 2, 2, 4, 1
-#define CFG_SMALL 256, 128, 64, 2, 4, 2, 1
-#elif NOISE_GEMM_CFG == 3
-#define CFG_BIG 256, 256, 32, 3, 2, 4, 1
-#define CFG_SMALL 256, 128, 32, 3, 4, 2, 1
-#elif NOISE_GEMM_CFG == 5
-#define CFG_BIG 256, 128, 32, 3, 2, 2, 2
-#define CFG_SMALL 256, 128, 32, 3, 2, 2, 2
-#elif NOISE_GEMM_CFG == 6
-#define CFG_BIG 256, 128, 32, 2, 2, 2, 2
-#define CFG_SMALL 256, 128, 32, 2, 2, 2, 2
-#elif NOISE_GEMM_CFG == 7
-#define CFG_BIG 128, 256, 32, 3, 2, 2, 2
-#define CFG_SMALL 128, 128, 32, 4, 2, 2, 2
-#endif
+#define CFG_WIDE 256, 128, 32, 4, 4, 2, 1
+#define CFG_MID 128, 128, 32, 4, 2, 2, 2
+#define CFG_SMALL 64, 64, 32, 4, 4, 1, 4
 
 template <int BM, int BN, int BK, int STAGES, int WGM, int WGN, int OCC>
 constexpr int cfg_wave_n() { return BN / WGN; }
@@ -636,10 +620,36 @@ int launch_cfg(const LowrankGemmArgs& g, hipStream_t stream) {
 
 bool use_big(int N) { return N % 256 == 0; }
 
+// The configuration of a launch, by how its tiles fill the CUs. Every configuration contracts K in the same order and
+// rounds alike, so the choice never changes a result.
+//  - 64 x 64 tiles while at most three of them fall on a CU: a larger tile then leaves most CUs idle behind one long K
+//    chain (2048 x 512 outputs, K = 2048: 42.9 us on 16 tiles of 256 x 256, 20.9 on 64 of 128 x 128, 10.7 on 256 of
+//    64 x 64; 6144 rows, three per CU: 43.4, 22.2, 20.4; 8192 rows, four per CU: 43.7, 23.3, 25.9).
+//  - beyond that, the fewer rounds of the GPU. In units of one round of 256 x 256 tiles (one workgroup per CU, 55.7 us
+//    at K = 2048), 128 x 128 tiles, two workgroups per CU, cost 0.585 a full round and 0.36 where the last one leaves
+//    one per CU; 256 x 128 tiles (N not a multiple of 256) 0.56. So 128 x 128 tiles run ragged ends (16384 rows: 47.4
+//    -> 34.7 us; 38400: 152 -> 134) and 256 x 256 ones every large launch (65536 rows: 146 against 118 us).
+enum class Tile { BIG, WIDE, MID, SMALL };
+Tile pick_tile(int M, int N) {
+  const long cus = num_cus();
+  const auto tiles = [&](long bm, long bn) { return (M + bm - 1) / bm * ((N + bn - 1) / bn); };
+  if (tiles(64, 64) <= 3 * cus) return Tile::SMALL;
+  const long mid = tiles(128, 128), rest = mid % (2 * cus);
+  const double mid_cost = mid / (2 * cus) * 0.585 + (rest > cus ? 0.585 : rest ? 0.36 : 0.);
+  const long wide = tiles(256, use_big(N) ? 256 : 128);
+  const double cost = (wide + cus - 1) / cus * (use_big(N) ? 1. : 0.56);
+  return mid_cost < cost ? Tile::MID : use_big(N) ? Tile::BIG : Tile::WIDE;
+}
+
 template <int EPI>
 int launch_epi(const LowrankGemmArgs& g, hipStream_t stream) {
-  if (use_big(g.N)) return launch_cfg<CFG_BIG, EPI>(g, stream);
-  return launch_cfg<CFG_SMALL, EPI>(g, stream);
+  // (EPI_QKV serves token counts that are no multiple of 32: one configuration per width)
+  const Tile t = EPI == EPI_QKV ? (use_big(g.N) ? Tile::BIG : Tile::WIDE) : pick_tile(g.M, g.N);
+  if constexpr (EPI != EPI_QKV) {
+    if (t == Tile::SMALL) return launch_cfg<CFG_SMALL, EPI>(g, stream);
+    if (t == Tile::MID) return launch_cfg<CFG_MID, EPI>(g, stream);
+  }
+  return t == Tile::BIG ? launch_cfg<CFG_BIG, EPI>(g, stream) : launch_cfg<CFG_WIDE, EPI>(g, stream);
 }
 
 }  // namespace
@@ -731,7 +741,7 @@ int head_weight_f16_launch(const float* w, long ldw, const float* gain, int N, i
 
 int lowrank_gemm_parts(int N) {
   if (N <= 0 || N % 128) return 0;
-  return use_big(N) ? N / cfg_wave_n<CFG_BIG>() : N / cfg_wave_n<CFG_SMALL>();
+  return use_big(N) ? N / cfg_wave_n<CFG_BIG>() : N / cfg_wave_n<CFG_WIDE>();
 }
 
 int lowrank_gemm_launch(int epi, const LowrankGemmArgs& g, hipStream_t stream) {

@@ -43,3 +43,62 @@ def test_weight_resident_product_from_both_weight_layouts(members, T, dout):
     ref = xd @ wd.t()
     bound = 2 ** -8 * ref.abs() + 512 * 2 ** -24 * (xd.abs() @ wd.abs().t())
     assert ((rows.cpu().double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize('out', ['f32', 'bf16', 'accumulate'])
+@pytest.mark.parametrize('dout,din,T', [(512, 576, 1000), (640, 128, 1000), (512, 2048, 250)])
+def test_tile_configurations_of_the_linear_agree_bit_for_bit(dout, din, T, out):
+    """The tile GEMM takes 64 x 64, 128 x 128 or the large tiles by the number of rows. Every member's rows are the same
+    bits whichever it takes: 48,000 rows (256 x 256 or, at 640 columns, 256 x 128 tiles), the first quarter of them
+    (128 x 128), and slices of up to 5,000 rows down to one member (64 x 64). T = 1000 and 250 leave ragged last tiles
+    and tiles that straddle members."""
+    from noise_amd import ops
+    g = torch.Generator().manual_seed(32)
+    P = 48000 // T
+    log_case(f'linear tile configurations {din}->{dout} T={T} {out}')
+    x = torch.randn(P, T, din, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(dout, din, generator=g) * din ** -0.5).bfloat16().to(DEV)
+    a, b = torch.randn(P, dout, generator=g).to(DEV), torch.randn(P, din, generator=g).to(DEV)
+    sign = (1e-2 * torch.randn(P, generator=g)).to(DEV)
+    res = torch.randn(P, T, dout, generator=g).to(DEV) if out == 'accumulate' else None
+
+    def run(lo, hi):
+        kw = dict(out=res[lo:hi].clone(), accumulate=True) if out == 'accumulate' else \
+            dict(out_dtype=torch.bfloat16 if out == 'bf16' else torch.float32)
+        return ops.lowrank_linear(x[lo:hi], w, a[lo:hi], b[lo:hi], sign[lo:hi], **kw)
+    whole = run(0, P)
+    for lo, hi in ((0, P // 4), (1, 1 + 5000 // T), (P - 1, P)):
+        assert torch.equal(run(lo, hi), whole[lo:hi]), (lo, hi)
+
+
+@pytest.mark.parametrize('T', [256, 250])
+@pytest.mark.parametrize('head', ['fp32', 'bf16', 'fp32_split'])
+def test_tile_configurations_of_the_head_agree_bit_for_bit(head, T):
+    """The same for the head's per-token losses: 16,384 rows (256 x 256 tiles), 2,560 (128 x 128) and one member
+    (64 x 64), from tiled operands (T = 256) and row-major ones with straddling tiles (T = 250)."""
+    from noise_amd.population import HEAD_FORMAT
+    g = torch.Generator().manual_seed(33)
+    P, V, fmt = 64, 4096, HEAD_FORMAT[head]
+    log_case(f'head tile configurations {head} T={T}')
+    x = torch.randn(P * T, 512, generator=g).to(DEV)
+    w = (torch.randn(V, 512, generator=g) * 0.05).to(DEV)
+    op = w
+    if head != 'fp32':
+        op = torch.empty(V, 1536 if head == 'fp32_split' else 512, device=DEV, dtype=torch.bfloat16)
+        _lib.call('noise_cast_bf16', w.data_ptr(), op.data_ptr(), w.numel(), 512 if head == 'fp32_split' else 0, _stream())
+    a, b = torch.randn(P, V, generator=g).to(DEV), torch.randn(P, 512, generator=g).to(DEV)
+    sign = (1e-2 * torch.randn(P, generator=g)).to(DEV)
+    tgt = torch.randint(0, V, (T,), generator=g).to(DEV)
+
+    def run(lo, hi):
+        m = hi - lo
+        n = _lib.size_query('noise_head_ce_workspace_size', m, T, V, fmt)
+        ws, loss = torch.empty(n, device=DEV, dtype=torch.uint8), torch.empty(m * T, device=DEV)
+        _lib.call('noise_head_ce', x[lo * T:].data_ptr(), 0, None, op.data_ptr(), V, fmt, a[lo:].data_ptr(),
+                  b[lo:].data_ptr(), sign[lo:].data_ptr(), tgt.data_ptr(), 0, m, T, 0, _lib.CE_NONE, loss.data_ptr(),
+                  None, ws.data_ptr(), n, None, 0, _stream())
+        torch.cuda.synchronize()
+        return loss
+    whole = run(0, P)
+    for lo, hi in ((4, 14), (P - 1, P)):
+        assert torch.equal(run(lo, hi), whole[lo * T:hi * T]), (lo, hi)
