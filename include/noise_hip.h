@@ -207,6 +207,14 @@ int noise_attention_noalloc(const void* qkv, int members, int T, int window, int
                             const float* b_proj, int pair_shift, void* y, float* upart, float* mom,
                             noise_stream_t stream);
 
+/* The same attention on separate operands (utils/model.py:24-31 as the credit reruns call it, train/val/run.py:618-622):
+ * q, k and v are 16-bit rows of 512 (8 heads x 64), 16-byte aligned, in q_blocks, k_blocks and v_blocks consecutive
+ * blocks of T rows; member p reads block p % blocks of each, so an operand that members share (the reruns' fixed heads
+ * and values: one block per batch row, members ordered draw by draw) is stored once. Each count divides members. No
+ * c_proj dots and no moments. */
+int noise_attention_heads(const void* q, int q_blocks, const void* k, int k_blocks, const void* v, int v_blocks,
+                          int members, int T, int window, int qk_norm, int qk_format, void* y, noise_stream_t stream);
+
 /* resid += lowrank(x, w) with the input-side dot of row r given as u_parts partial sums
  * u[r * u_row_stride + q * u_part_stride]: the attention c_proj (u from noise_attention: row stride 8,
  * part stride 1) and the MLP c_proj (u from noise_mlp_fc: row stride 1, part stride members*T).

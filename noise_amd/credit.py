@@ -31,6 +31,18 @@ def _tables(t, T):
     return t.float().contiguous()
 
 
+def _rows(t):
+    """t as contiguous bf16 rows at a 16-byte address, which the attention kernel reads in place: the tensor itself when
+    it is."""
+    t = t.to(torch.bfloat16).contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _value_rows(t):
+    """The bf16-rounded values in fp16, the kernel's operand format."""
+    return t.to(torch.bfloat16).to(torch.float16, memory_format=torch.contiguous_format)
+
+
 def moved_heads(raw, a, sigma, cos, sin):
     """norm(rotary(raw + sigma a)) per draw, flattened over (draw, batch): [n * b, t, h, 64] in a's dtype
     (bf16) (train/val/run.py:186-189)."""
@@ -111,22 +123,19 @@ def attention(q, k, v, window, qk_norm=False):
         raise ValueError(f'the attention kernel runs whole 128-token blocks: token count {T} is not a multiple of 128')
     for t, nm in ((q, 'q'), (k, 'k'), (v, 'v')):
         _cuda(t, nm)
-    qkv = torch.empty(B * T, 3 * H * HD, device=q.device, dtype=torch.bfloat16)
-    qkv[:, :H * HD] = q.reshape(B * T, H * HD).to(torch.bfloat16)
-    qkv[:, H * HD:2 * H * HD] = k.reshape(B * T, H * HD).to(torch.bfloat16)
-    qkv[:, 2 * H * HD:] = v.reshape(B * T, H * HD).to(torch.bfloat16).half().view(torch.bfloat16)
+    q, k, v = _rows(q), _rows(k), _value_rows(v)
     y = torch.empty(B * T, H * HD, device=q.device, dtype=torch.bfloat16)
-    _lib.call('noise_attention', qkv.data_ptr(), B, T, int(window), int(bool(qk_norm)), _lib.QK_BF16, None, 0,
-              y.data_ptr(), None, None, None, 0, _stream())
+    _lib.call('noise_attention_heads', q.data_ptr(), B, k.data_ptr(), B, v.data_ptr(), B, B, T, int(window),
+              int(bool(qk_norm)), _lib.QK_BF16, y.data_ptr(), _stream())
     return y.view(B, T, H, HD)
 
 
 def rerun(kind, raw, a, sigma, cos, sin, fixed, values, window):
-    """The attention reruns of one chunk of draws in `query_key_errors` (train/val/run.py:618-622): the moved
-    heads of `kind` ('q' or 'k') are written straight into their slot of the q | k | v rows the attention kernel
-    reads, beside the other processed head `fixed` and `values` (both [b, t, h, 64], shared by every draw).
-    Returns the attention output [n, b, t, h, 64] bf16. Both head slots hold RMS-normalised rows, so the kernel
-    runs with bounded scores (no running maximum)."""
+    """The attention reruns of one chunk of draws in `query_key_errors` (train/val/run.py:618-622): the moved heads of
+    `kind` ('q' or 'k') against the other processed head `fixed` and `values` (both [b, t, h, 64]), which every draw
+    reads from the one copy (64 draws of 2048 tokens: the broadcast copies beside each draw's moved heads took 202 us,
+    and the moved heads' own rows 68 instead of 42). Returns the attention output [n, b, t, h, 64] bf16. Both heads hold
+    RMS-normalised rows, so the kernel runs with bounded scores (no running maximum)."""
     if kind not in ('q', 'k'):
         raise ValueError("kind must be 'q' or 'k'")
     n, b, T, H, hd = a.shape
@@ -143,17 +152,17 @@ def rerun(kind, raw, a, sigma, cos, sin, fixed, values, window):
     cos, sin = _tables(cos, T), _tables(sin, T)
     _cuda(raw, 'raw'), _cuda(a, 'a'), _cuda(fixed, 'fixed'), _cuda(values, 'values')
     W = H * HD
-    moved_slot, fixed_slot = (0, W) if kind == 'q' else (W, 0)
-    qkv = torch.empty(n, b * T, 3 * W, device=a.device, dtype=torch.bfloat16)
-    qkv[:, :, fixed_slot:fixed_slot + W] = fixed.reshape(1, b * T, W).to(torch.bfloat16)
-    qkv[:, :, 2 * W:] = values.reshape(1, b * T, W).to(torch.bfloat16).half().view(torch.bfloat16)
+    moved = torch.empty(n * b * T, W, device=a.device, dtype=torch.bfloat16)
+    fixed, values = _rows(fixed), _value_rows(values)
     rawf, a = raw.float().contiguous(), a.contiguous()
     stream = _stream()
     _lib.call('noise_moved_heads', rawf.data_ptr(), a.data_ptr(), float(sigma), cos.data_ptr(), sin.data_ptr(), n, b,
-              T, H, qkv.data_ptr() + 2 * moved_slot, 3 * W, stream)
+              T, H, moved.data_ptr(), W, stream)
+    # every draw reads the same b blocks of fixed heads and values
+    q, k = ((moved, n * b), (fixed, b)) if kind == 'q' else ((fixed, b), (moved, n * b))
     y = torch.empty(n * b * T, W, device=a.device, dtype=torch.bfloat16)
-    _lib.call('noise_attention', qkv.data_ptr(), n * b, T, int(window), 1, _lib.QK_BF16, None, 0, y.data_ptr(), None,
-              None, None, 0, stream)
+    _lib.call('noise_attention_heads', q[0].data_ptr(), q[1], k[0].data_ptr(), k[1], values.data_ptr(), b, n * b, T,
+              int(window), 1, _lib.QK_BF16, y.data_ptr(), stream)
     return y.view(n, b, T, H, HD)
 
 

@@ -304,10 +304,11 @@ int noise_attention(const void* qkv, int members, int T, int window, int qk_norm
   }
   if ((b_proj == nullptr) != (upart == nullptr)) return NOISE_EINVAL;
   AttnArgs g{};
-  g.qkv = static_cast<const bf16*>(qkv);
-  g.ldq = 3 * DM;
-  g.koff = DM;
-  g.voff = 2 * DM;
+  const bf16* rows = static_cast<const bf16*>(qkv);
+  if (!rows) return NOISE_EINVAL;
+  g.q = {rows, 3 * DM, members};
+  g.k = {rows + DM, 3 * DM, members};
+  g.v = {rows + 2 * DM, 3 * DM, members};
   g.y = static_cast<bf16*>(y);
   g.ldy = DM;
   g.members = members;
@@ -341,6 +342,26 @@ int noise_attention_noalloc(const void* qkv, int members, int T, int window, int
   // the same kernels as noise_attention; every partial is written before it is read, so nothing is cleared
   return noise_attention(qkv, members, T, window, qk_norm, qk_format, b_proj, pair_shift, y, upart, mom, work, bytes,
                          stream);
+}
+
+int noise_attention_heads(const void* q, int q_blocks, const void* k, int k_blocks, const void* v, int v_blocks,
+                          int members, int T, int window, int qk_norm, int qk_format, void* y, noise_stream_t stream) {
+  if (bad_members(members, T, 0)) return NOISE_EINVAL;
+  for (const int blocks : {q_blocks, k_blocks, v_blocks})
+    if (blocks <= 0 || members % blocks) return NOISE_EINVAL;
+  AttnArgs g{};
+  g.q = {static_cast<const bf16*>(q), DM, q_blocks};
+  g.k = {static_cast<const bf16*>(k), DM, k_blocks};
+  g.v = {static_cast<const bf16*>(v), DM, v_blocks};
+  g.y = static_cast<bf16*>(y);
+  g.ldy = DM;
+  g.members = members;
+  g.T = T;
+  g.H = NH;
+  g.window = window;
+  g.qk_norm = qk_norm != 0;
+  g.qk_format = qk_format;
+  return attention_launch(g, static_cast<hipStream_t>(stream));
 }
 
 int noise_lowrank_resid(const void* x, const void* w, int in, int out, const float* a, const float* u, int u_parts,

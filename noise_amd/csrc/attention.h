@@ -6,11 +6,15 @@
 // QK_BF16_V_BF16: q, k and v bf16 and the probabilities rounded to bf16 for P V (torch's bf16 attention operands)
 enum : int { QK_BF16 = 0, QK_F16 = 1, QK_F16_Q_LOG2 = 2, QK_BF16_V_BF16 = 3 };
 
+// One of q, k, v: 16-bit rows of ld elements, head h at columns h*64 .. h*64+63 of row t of its member block. Member p
+// reads block p % period: period = members for rows of its own, fewer where members share them (the credit reruns'
+// fixed heads and values, one block per batch row).
+struct AttnHeads {
+  const __bf16* p;
+  int ld, period;
+};
 struct AttnArgs {
-  const __bf16* qkv;  // [members * T, ldq] 16-bit rows; q at column h*64, k at koff + h*64, v (fp16; bf16 for QK_BF16_V_BF16) at
-                      // voff + h*64
-  long ldq;
-  int koff, voff;
+  AttnHeads q, k, v;  // v fp16 (bf16 for QK_BF16_V_BF16)
   __bf16* y;          // [members * T, ldy], head h at columns h*64 .. h*64+63
   long ldy;
   int members, T, H, window;

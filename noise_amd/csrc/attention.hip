@@ -152,8 +152,12 @@ __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
   const int ph = (int)(n / nq), qblk = nq - 1 - (int)(n % nq), h = ph % g.H, p = ph / g.H;
   const int q0 = qblk * BQ;
   const long rbase = (long)p * g.T;
-  const bf16* qkv = g.qkv;
-  const int qcol = h * HD, kcol = g.koff + h * HD, vcol = g.voff + h * HD;
+  // the member's block of each operand, at this head's columns (the division only where members share blocks)
+  auto heads = [&](const AttnHeads& o) {
+    const int blk = p < o.period ? p : p % o.period;
+    return o.p + (long)blk * g.T * o.ld + h * HD;
+  };
+  const bf16 *qh = heads(g.q), *kh = heads(g.k), *vh = heads(g.v);
 
   // Q fragments (MFMA B operand): query q0 + 32 wave + 16 qb + lane % 16, dims 32 kk + 8 grp ..
   bf16x8 qf[2][2];
@@ -162,7 +166,7 @@ __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
       qf[qb][kk] = *reinterpret_cast<const bf16x8*>(
-          qkv + (rbase + q0 + 32 * wave + 16 * qb + (lane & 15)) * g.ldq + qcol + 32 * kk + 8 * grp);
+          qh + (long)(q0 + 32 * wave + 16 * qb + (lane & 15)) * g.q.ld + 32 * kk + 8 * grp);
 
   const int k_lo = max(0, q0 - g.window), k_hi = min(g.T - 1, q0 + BQ - 1);
   const int j0 = k_lo / BKV, j1 = k_hi / BKV;
@@ -175,17 +179,17 @@ __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
 #pragma unroll
   for (int q = 0; q < DH; ++q) {
     const int R = 8 * (DH * wave + q) + lrow;
-    koffs[q] = 2u * (unsigned)(key_of_krow(R) * g.ldq + kcol + 8 * (lchunk ^ (R & 7)));
-    voffs[q] = 2u * (unsigned)(R * g.ldq + vcol + 8 * (lchunk ^ vsw(R)));
+    koffs[q] = 2u * (unsigned)(key_of_krow(R) * g.k.ld + 8 * (lchunk ^ (R & 7)));
+    voffs[q] = 2u * (unsigned)(R * g.v.ld + 8 * (lchunk ^ vsw(R)));
   }
   auto issue = [&](int j, int buf) {
-    const bf16* kv0 = qkv + (rbase + (long)j * BKV) * g.ldq;
+    const bf16 *k0 = kh + (long)j * BKV * g.k.ld, *v0 = vh + (long)j * BKV * g.v.ld;
 #pragma unroll
     for (int q = 0; q < DH; ++q)
-      dma_x4_s(kv0, koffs[q], reinterpret_cast<const char*>(sk[buf]) + (DH * wave + q) * 1024);
+      dma_x4_s(k0, koffs[q], reinterpret_cast<const char*>(sk[buf]) + (DH * wave + q) * 1024);
 #pragma unroll
     for (int q = 0; q < DH; ++q)
-      dma_x4_s(kv0, voffs[q], reinterpret_cast<const char*>(sv[buf]) + (DH * wave + q) * 1024);
+      dma_x4_s(v0, voffs[q], reinterpret_cast<const char*>(sv[buf]) + (DH * wave + q) * 1024);
   };
 
   const float c2 = QL2 ? 1.f : 0.125f * 1.4426950408889634f;  // scores -> log2 units: 1/sqrt(64) * log2(e)
@@ -409,9 +413,13 @@ __global__ void moments_reduce_kernel(const float* part, float* out, int nqb, in
 long attention_moment_partials(int members, int T, int H) { return (long)members * H * (T / BQ) * 2 * HD; }
 
 int attention_launch(const AttnArgs& g, hipStream_t s) {
-  if (!g.qkv || !g.y || g.members <= 0 || g.T <= 0 || g.T % BQ || g.T % BKV || g.H <= 0 || g.window < 0 ||
-      g.ldq % 8 || g.ldy % 8 || g.koff % 8 || g.voff % 8 || ((uintptr_t)g.qkv & 15) || ((uintptr_t)g.y & 15))
+  if (!g.y || g.members <= 0 || g.T <= 0 || g.T % BQ || g.T % BKV || g.H <= 0 || g.window < 0 || g.ldy % 8 ||
+      ((uintptr_t)g.y & 15))
     return NOISE_EINVAL;
+  for (const AttnHeads* o : {&g.q, &g.k, &g.v})
+    // (the kernel's byte offsets inside a 64-key block are 32-bit)
+    if (!o->p || o->period <= 0 || o->ld < g.H * HD || o->ld % 8 || o->ld > (1 << 20) || ((uintptr_t)o->p & 15))
+      return NOISE_EINVAL;
   if (g.upart && (!g.b_proj || g.upart_ld < g.H || g.b_ld < g.H * HD)) return NOISE_EINVAL;
   if (g.mom && !g.mom_out) return NOISE_EINVAL;
   if (g.qk_format < QK_BF16 || g.qk_format > QK_BF16_V_BF16 ||

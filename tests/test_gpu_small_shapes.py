@@ -102,3 +102,47 @@ def test_tile_configurations_of_the_head_agree_bit_for_bit(head, T):
     whole = run(0, P)
     for lo, hi in ((4, 14), (P - 1, P)):
         assert torch.equal(run(lo, hi), whole[lo * T:hi * T]), (lo, hi)
+
+
+@pytest.mark.parametrize('shared', ['q', 'k'])
+@pytest.mark.parametrize('qk_norm', [0, 1])
+def test_attention_on_shared_heads_equals_packed_rows(shared, qk_norm):
+    """Attention on separate operands, one of q and k and the values stored once per batch row for every draw, is bit for
+    bit the attention on packed q | k | v rows that hold a copy per member."""
+    g = torch.Generator().manual_seed(34)
+    n, b, T, window = 3, 2, 256, 100
+    log_case(f'attention on shared heads: {shared} shared, qk_norm={qk_norm}')
+
+    def heads(blocks):
+        x = torch.randn(blocks * T, 8, 64, generator=g)
+        return (x * torch.rsqrt(x.square().mean(-1, keepdim=True))).view(blocks * T, 512).bfloat16().to(DEV)
+    own, fixed = heads(n * b), heads(b)
+    v = torch.randn(b * T, 512, generator=g).bfloat16().half().to(DEV)
+    q, k = ((fixed, b), (own, n * b)) if shared == 'q' else ((own, n * b), (fixed, b))
+    y = torch.empty(n * b * T, 512, device=DEV, dtype=torch.bfloat16)
+    _lib.call('noise_attention_heads', q[0].data_ptr(), q[1], k[0].data_ptr(), k[1], v.data_ptr(), b, n * b, T, window,
+              qk_norm, _lib.QK_BF16, y.data_ptr(), _stream())
+    rows = torch.cat([t[0].repeat(n * b // t[1], 1) for t in (q, k, (v.view(torch.bfloat16), b))], 1).contiguous()
+    ref = torch.empty_like(y)
+    _lib.call('noise_attention', rows.data_ptr(), n * b, T, window, qk_norm, _lib.QK_BF16, None, 0, ref.data_ptr(), None,
+              None, None, 0, _stream())
+    torch.cuda.synchronize()
+    assert torch.equal(y, ref)
+
+
+def test_credit_attention_of_strided_misaligned_and_float_heads():
+    """credit.attention reads contiguous aligned bf16 heads in place; transposed, offset and fp32 ones give the same."""
+    from noise_amd import credit
+    g = torch.Generator().manual_seed(35)
+    B, T = 2, 128
+    log_case('credit.attention of strided, misaligned and fp32 heads')
+    q, k, v = (torch.randn(B, T, 8, 64, generator=g).bfloat16().to(DEV) for _ in range(3))
+    ref = credit.attention(q, k, v, 50)
+
+    def strided(t):
+        return t.transpose(1, 2).contiguous().transpose(1, 2)
+
+    def shifted(t):
+        return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+    for f in (strided, shifted, torch.Tensor.float):
+        assert torch.equal(credit.attention(f(q), f(k), f(v), 50), ref), f
