@@ -11,8 +11,8 @@
 // torch's bf16 autocast rounding (the speedrun's scorer, utils/eval.py:44-45) runs it on bf16 q, k and v with the
 // probabilities rounded to bf16 for P V, as torch's attention on bf16 operands does.
 //
-// One workgroup = one (member, head, 128-query block); 4 waves of 32 queries; four workgroups per CU (122
-// VGPRs, 34 KiB of LDS each: 4 waves per SIMD hide the LDS and transcendental latencies).
+// One workgroup = one (member, head, 128-query block); 4 waves of 32 queries (64 queries, 16 per wave, in small grids);
+// four workgroups per CU (122 VGPRs, 34 KiB of LDS each: 4 waves per SIMD hide the LDS and transcendental latencies).
 // K/V blocks of 64 keys go through a double-buffered LDS ring filled by direct global -> LDS loads
 // (global_load_lds_dwordx4, issued from inline assembly so the compiler adds no LDS-wide waits): while block j
 // is computed, block j + 1 lands; one s_waitcnt vmcnt(0) + s_barrier per block (the loads are the only
@@ -41,7 +41,7 @@
 
 namespace {
 
-constexpr int HD = 64, BQ = 128, BKV = 64, NWAVE = 4, NTH = NWAVE * 64;
+constexpr int HD = 64, BQ_MAX = 128, BKV = 64, NWAVE = 4, NTH = NWAVE * 64;
 constexpr int DH = BKV * HD * 2 / 1024 / NWAVE;  // K (and V) load instructions per wave and block
 constexpr int KB = BKV / 16;       // 16-key MFMA blocks per key block
 constexpr int KC = BKV / 32;       // 32-key contraction steps of P V
@@ -124,8 +124,10 @@ __device__ __forceinline__ unsigned pack2(float a, float b) {
 // and the softmax takes exp2 of them directly: one VALU multiply per score less (with QKN no max is subtracted).
 // VB: v is bf16 and the probabilities are rounded to bf16 for P V (the operands of torch's attention on bf16 q, k, v:
 // the autocast clean forward); fp16 otherwise.
-template <bool QKN, bool F16, bool QL2, bool VB>
+// QB: 16-query blocks per wave (a workgroup has 64 QB queries); see attention_launch for the choice.
+template <bool QKN, bool F16, bool QL2, bool VB, int QB>
 __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
+  constexpr int BQ = 64 * QB;
   static_assert(!QL2 || QKN, "pre-scaled q is the population forward's QK-normalised format");
   static_assert(!VB || !F16, "bf16 v comes with bf16 q and k");
   // element type of v and of the probabilities
@@ -160,13 +162,13 @@ __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
   const bf16 *qh = heads(g.q), *kh = heads(g.k), *vh = heads(g.v);
 
   // Q fragments (MFMA B operand): query q0 + 32 wave + 16 qb + lane % 16, dims 32 kk + 8 grp ..
-  bf16x8 qf[2][2];
+  bf16x8 qf[QB][2];
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb)
+  for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
       qf[qb][kk] = *reinterpret_cast<const bf16x8*>(
-          qh + (long)(q0 + 32 * wave + 16 * qb + (lane & 15)) * g.q.ld + 32 * kk + 8 * grp);
+          qh + (long)(q0 + 16 * QB * wave + 16 * qb + (lane & 15)) * g.q.ld + 32 * kk + 8 * grp);
 
   const int k_lo = max(0, q0 - g.window), k_hi = min(g.T - 1, q0 + BQ - 1);
   const int j0 = k_lo / BKV, j1 = k_hi / BKV;
@@ -193,14 +195,17 @@ __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
   };
 
   const float c2 = QL2 ? 1.f : 0.125f * 1.4426950408889634f;  // scores -> log2 units: 1/sqrt(64) * log2(e)
-  float mref[2] = {-1e30f, -1e30f};  // running max (score units)
+  float mref[QB];  // running max (score units)
   // O^T accumulators, and the row sums of the fp16 probabilities actually used in P V, accumulated on the
   // MFMA pipe (an all-ones A operand: every element of osum[qb] in lane l is the sum for query l % 16)
-  f32x4 o[2][4], osum[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+  f32x4 o[QB][4], osum[QB];
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb)
+  for (int qb = 0; qb < QB; ++qb) {
+    mref[qb] = -1e30f;
+    osum[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int db = 0; db < 4; ++db) o[qb][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 
   // per-lane LDS offsets of the MFMA operand reads (the block / step index adds a constant)
   // K block kb: row 16 kb + lane % 16, chunk grp and 4 + grp
@@ -236,17 +241,17 @@ __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
         sq[kb][e] = keep_ge ? select_lanes(sq[kb][e], neg_inf, m) : select_lanes(neg_inf, sq[kb][e], m);
       }
   };
-  auto apply_mask = [&](f32x4 (&s)[2][KB], int kstart, bool causal_edge, bool window_edge) {
+  auto apply_mask = [&](f32x4 (&s)[QB][KB], int kstart, bool causal_edge, bool window_edge) {
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
-      const int t0 = kstart - q0 - 32 * wave - 16 * qb;
+    for (int qb = 0; qb < QB; ++qb) {
+      const int t0 = kstart - q0 - 16 * QB * wave - 16 * qb;
       // causal: keep the lanes with v >= t; window: drop the lanes with v >= t + window + 1
       if (causal_edge) mask_edge(s[qb], t0, true);
       if (window_edge) mask_edge(s[qb], t0 + g.window + 1, false);
     }
   };
   // Online softmax of one key block for query block qb of this wave.
-  auto softmax = [&](f32x4 (&s)[2][KB], pt8 (&pf)[2][KC], int qb) {
+  auto softmax = [&](f32x4 (&s)[QB][KB], pt8 (&pf)[QB][KC], int qb) {
     float mc = 0.f;
     if constexpr (!QKN) {
       float m0 = -INFINITY, m1 = -INFINITY;
@@ -288,13 +293,13 @@ __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
     const bf16* kt = sk[buf];
     const char* vt = reinterpret_cast<const char*>(sv[buf]);
     // S^T = K Q^T
-    f32x4 s[2][KB];
+    f32x4 s[QB][KB];
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
       const bf16x8 k0 = *reinterpret_cast<const bf16x8*>(&kt[kofs0 + 1024 * kb]);
       const bf16x8 k1 = *reinterpret_cast<const bf16x8*>(&kt[kofs1 + 1024 * kb]);
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) {
+      for (int qb = 0; qb < QB; ++qb) {
         f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
         a = mfma_qk<F16>(k0, qf[qb][0], a);
         s[qb][kb] = mfma_qk<F16>(k1, qf[qb][1], a);
@@ -303,9 +308,9 @@ __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
     // blocks away from the causal edge and the window edge need no mask
     const bool causal_edge = kstart + BKV - 1 > q0, window_edge = q0 + BQ - 1 - kstart > g.window;
     if (causal_edge || window_edge) apply_mask(s, kstart, causal_edge, window_edge);
-    pt8 pf[2][KC];
-    softmax(s, pf, 0);
-    softmax(s, pf, 1);
+    pt8 pf[QB][KC];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) softmax(s, pf, qb);
     // O^T += V^T P^T
 #pragma unroll
     for (int c = 0; c < KC; ++c)
@@ -316,12 +321,12 @@ __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
         const pt4 lo16 = __builtin_bit_cast(pt4, lo), hi16 = __builtin_bit_cast(pt4, hi);
         const pt8 vf = {lo16[0], lo16[1], lo16[2], lo16[3], hi16[0], hi16[1], hi16[2], hi16[3]};
 #pragma unroll
-        for (int qb = 0; qb < 2; ++qb) o[qb][db] = mfma_pv(vf, pf[qb][c], o[qb][db]);
+        for (int qb = 0; qb < QB; ++qb) o[qb][db] = mfma_pv(vf, pf[qb][c], o[qb][db]);
       }
 #pragma unroll
     for (int c = 0; c < KC; ++c)
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) osum[qb] = mfma_pv(ones, pf[qb][c], osum[qb]);
+      for (int qb = 0; qb < QB; ++qb) osum[qb] = mfma_pv(ones, pf[qb][c], osum[qb]);
     // block j + 1 has landed for this wave (the only vector memory operations in flight are its loads);
     // the barrier makes every wave's part visible and retires slot buf
     __builtin_amdgcn_s_waitcnt(0);
@@ -344,9 +349,9 @@ __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
 #pragma unroll
   for (int e = 0; e < 16; ++e) mom1[e] = mom2[e] = 0.f;
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
+  for (int qb = 0; qb < QB; ++qb) {
     const float inv = 1.f / osum[qb][0];
-    const int q = q0 + 32 * wave + 16 * qb + (lane & 15);
+    const int q = q0 + 16 * QB * wave + 16 * qb + (lane & 15);
     const long row = rbase + q;
     // yv[4 db + e] is dim 16 db + 4 grp + e
     float yv[16];
@@ -375,7 +380,7 @@ __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
       mom2[e] += yv[e] * yv[e];
     }
   }
-  if (g.mom) {
+  if (QB == 2 && g.mom) {
     // sum over the wave's 32 queries (lanes sharing lane / 16), then over the 4 waves
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
@@ -410,10 +415,10 @@ __global__ void moments_reduce_kernel(const float* part, float* out, int nqb, in
 
 }  // namespace
 
-long attention_moment_partials(int members, int T, int H) { return (long)members * H * (T / BQ) * 2 * HD; }
+long attention_moment_partials(int members, int T, int H) { return (long)members * H * (T / BQ_MAX) * 2 * HD; }
 
 int attention_launch(const AttnArgs& g, hipStream_t s) {
-  if (!g.y || g.members <= 0 || g.T <= 0 || g.T % BQ || g.T % BKV || g.H <= 0 || g.window < 0 || g.ldy % 8 ||
+  if (!g.y || g.members <= 0 || g.T <= 0 || g.T % BQ_MAX || g.T % BKV || g.H <= 0 || g.window < 0 || g.ldy % 8 ||
       ((uintptr_t)g.y & 15))
     return NOISE_EINVAL;
   for (const AttnHeads* o : {&g.q, &g.k, &g.v})
@@ -425,25 +430,37 @@ int attention_launch(const AttnArgs& g, hipStream_t s) {
   if (g.qk_format < QK_BF16 || g.qk_format > QK_BF16_V_BF16 ||
       ((g.qk_format == QK_F16_Q_LOG2 || g.qk_format == QK_BF16_V_BF16) && !g.qk_norm))
     return NOISE_EINVAL;
-  const long grid = (long)(g.T / BQ) * g.H * g.members;
+  const long grid = (long)(g.T / BQ_MAX) * g.H * g.members;
   if (grid > 0x7fffffffL) return NOISE_ENOTSUP;
-  if (g.qk_format == QK_F16_Q_LOG2)
-    hipLaunchKernelGGL((attention_kernel<true, true, true, false>), dim3((unsigned)grid), dim3(NTH), 0, s, g);
-  else if (g.qk_format == QK_BF16_V_BF16)
-    hipLaunchKernelGGL((attention_kernel<true, false, false, true>), dim3((unsigned)grid), dim3(NTH), 0, s, g);
-  else if (g.qk_norm && g.qk_format == QK_F16)
-    hipLaunchKernelGGL((attention_kernel<true, true, false, false>), dim3((unsigned)grid), dim3(NTH), 0, s, g);
-  else if (g.qk_norm)
-    hipLaunchKernelGGL((attention_kernel<true, false, false, false>), dim3((unsigned)grid), dim3(NTH), 0, s, g);
-  else if (g.qk_format == QK_F16)
-    hipLaunchKernelGGL((attention_kernel<false, true, false, false>), dim3((unsigned)grid), dim3(NTH), 0, s, g);
-  else
-    hipLaunchKernelGGL((attention_kernel<false, false, false, false>), dim3((unsigned)grid), dim3(NTH), 0, s, g);
+  // 64 queries per workgroup while 128-query ones would not fill the GPU twice: one workgroup then has a CU (almost) to
+  // itself and its serial chain of key blocks sets the time, which half the queries shorten (one 2048-token sequence,
+  // window 1024, 128 workgroups: 16.5 -> 10.6 us; 8 x 256 tokens 7.8 -> 5.4; 512 workgroups 24.0 -> 23.1). Up to four
+  // per CU also where causal chains of more than 1024 keys differ most in length (8 x 2048 tokens, window 2048: 57.6 ->
+  // 52.0; window 1024: 39.8 -> 40.5). Larger grids lose: the K/V blocks are read twice as often (64 members 101.8 ->
+  // 107.7). A query's key blocks and their order are the same either way, and so are its bits. The moments' partials
+  // are per 128 queries. (Deeper K/V rings, three blocks in flight, measured no gain at any grid.)
+  const long cus = num_cus();
+  const bool narrow = !g.mom && (grid <= 2 * cus || (grid <= 4 * cus && (g.window < g.T ? g.window : g.T) > 1024));
+  auto launch = [&](auto qkn, auto f16, auto ql2, auto vb) {
+    constexpr bool A = decltype(qkn)::value, B = decltype(f16)::value, C = decltype(ql2)::value, V = decltype(vb)::value;
+    if (narrow)
+      hipLaunchKernelGGL((attention_kernel<A, B, C, V, 1>), dim3((unsigned)(2 * grid)), dim3(NTH), 0, s, g);
+    else
+      hipLaunchKernelGGL((attention_kernel<A, B, C, V, 2>), dim3((unsigned)grid), dim3(NTH), 0, s, g);
+  };
+  const std::true_type yes{};
+  const std::false_type no{};
+  if (g.qk_format == QK_F16_Q_LOG2) launch(yes, yes, yes, no);
+  else if (g.qk_format == QK_BF16_V_BF16) launch(yes, no, no, yes);
+  else if (g.qk_norm && g.qk_format == QK_F16) launch(yes, yes, no, no);
+  else if (g.qk_norm) launch(yes, no, no, no);
+  else if (g.qk_format == QK_F16) launch(no, yes, no, no);
+  else launch(no, no, no, no);
   NOISE_CHECK_LAUNCH();
   if (g.mom) {
     const long n = (long)g.members * g.H * 2 * HD;
     hipLaunchKernelGGL(moments_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, g.mom, g.mom_out,
-                       g.T / BQ, g.T, n);
+                       g.T / BQ_MAX, g.T, n);
     NOISE_CHECK_LAUNCH();
   }
   return NOISE_OK;

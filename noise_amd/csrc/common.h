@@ -201,3 +201,15 @@ __device__ __forceinline__ void store_stream_x4(void* p, unsigned a, unsigned b,
 __device__ __forceinline__ void store_stream_f4(void* p, float a, float b, float c, float d) {
   store_stream_x4(p, u32x4{__float_as_uint(a), __float_as_uint(b), __float_as_uint(c), __float_as_uint(d)});
 }
+
+// Compute units of the current device (256 where it cannot be asked), looked up once.
+inline int num_cus() {
+  static int cus = [] {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+      n = 256;
+    return n;
+  }();
+  return cus;
+}

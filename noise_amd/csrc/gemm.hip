@@ -588,17 +588,6 @@ lowrank_gemm_kernel(const LowrankGemmArgs g) {
 template <int BM, int BN, int BK, int STAGES, int WGM, int WGN, int OCC>
 constexpr int cfg_wave_n() { return BN / WGN; }
 
-int num_cus() {
-  static int cus = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    return n;
-  }();
-  return cus;
-}
-
 template <int BM, int BN, int BK, int STAGES, int WGM, int WGN, int OCC, int EPI>
 int launch_cfg(const LowrankGemmArgs& g, hipStream_t stream) {
   using C = Cfg<BM, BN, BK, STAGES, WGM, WGN>;

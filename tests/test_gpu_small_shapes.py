@@ -146,3 +146,40 @@ def test_credit_attention_of_strided_misaligned_and_float_heads():
         return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
     for f in (strided, shifted, torch.Tensor.float):
         assert torch.equal(credit.attention(f(q), f(k), f(v), 50), ref), f
+
+
+@pytest.mark.parametrize('fmt,qk_norm', [(_lib.QK_F16_Q_LOG2, 1), (_lib.QK_BF16_V_BF16, 1), (_lib.QK_BF16, 1),
+                                         (_lib.QK_F16, 1), (_lib.QK_BF16, 0), (_lib.QK_F16, 0)])
+@pytest.mark.parametrize('T,window', [(128, 128), (384, 65), (1152, 1100)])
+def test_attention_of_64_and_128_queries_per_workgroup_agree_bit_for_bit(T, window, fmt, qk_norm):
+    """A small grid takes 64 queries per workgroup, a large one (or one with moments) 128: the first member's rows and
+    c_proj dots are the same bits alone, with moments, and among enough members to fill the GPU."""
+    g = torch.Generator(DEV).manual_seed(36)
+    m = 1 + 8 * 1024 // (T // 128 * 8)
+    log_case(f'attention 64 / 128 queries T={T} window={window} format={fmt} qk_norm={qk_norm}')
+    x = torch.randn(m * T, 3, 8, 64, device=DEV, generator=g)
+    if qk_norm:
+        x[:, :2] *= torch.rsqrt(x[:, :2].square().mean(-1, keepdim=True))
+    if fmt == _lib.QK_F16_Q_LOG2:
+        x[:, 0] *= 0.18033688
+    half = fmt in (_lib.QK_F16, _lib.QK_F16_Q_LOG2)
+    rows = x.half().view(torch.bfloat16) if half else x.bfloat16()
+    if fmt == _lib.QK_BF16:
+        rows[:, 2] = rows[:, 2].half().view(torch.bfloat16)
+    b = torch.randn(m, 512, device=DEV, generator=g)
+
+    def run(members, moments):
+        y = torch.empty(members * T, 512, device=DEV, dtype=torch.bfloat16)
+        u, mom = torch.empty(members * T, 8, device=DEV), torch.empty(members, 8, 2, 64, device=DEV)
+        n = _lib.size_query('noise_attention_workspace_size', members, T)
+        ws = torch.empty(n, device=DEV, dtype=torch.uint8)
+        _lib.call('noise_attention', rows.data_ptr(), members, T, window, qk_norm, fmt, b.data_ptr(), 0, y.data_ptr(),
+                  u.data_ptr(), mom.data_ptr() if moments else None, ws.data_ptr() if moments else None,
+                  n if moments else 0, _stream())
+        torch.cuda.synchronize()
+        return y[:T], u[:T]
+    alone = run(1, False)
+    for other in (run(1, True), run(m, False)):
+        assert torch.equal(alone[0], other[0]) and torch.equal(alone[1], other[1])
+    # (the same kernel's numbers against the oracle: test_attention_matches_oracle_and_moments)
+    assert torch.isfinite(alone[0].float()).all()
