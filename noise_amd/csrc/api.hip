@@ -625,14 +625,14 @@ int noise_adam_batch(const noise_adam_tensor_t* tensors, int n, float beta1, flo
   std::vector<AdamTensor> t(n);
   for (int k = 0; k < n; ++k)
     t[k] = AdamTensor{tensors[k].param, tensors[k].grad, tensors[k].exp_avg, tensors[k].exp_avg_sq, tensors[k].n,
-                      tensors[k].step_size, tensors[k].bc2_sqrt, 0};
+                      tensors[k].step_size, tensors[k].bc2_sqrt};
   return adam_batch_launch(t.data(), n, beta1, beta2, eps, static_cast<hipStream_t>(stream));
 }
 
 int noise_adam(float* param, const float* grad, float* exp_avg, float* exp_avg_sq, long n, float step_size,
                float beta1, float beta2, float eps, float bc2_sqrt, noise_stream_t stream) {
-  AdamArgs g{param, grad, exp_avg, exp_avg_sq, n, step_size, beta1, beta2, eps, bc2_sqrt};
-  return adam_launch(g, static_cast<hipStream_t>(stream));
+  const AdamTensor t{param, grad, exp_avg, exp_avg_sq, n, step_size, bc2_sqrt};
+  return adam_batch_launch(&t, 1, beta1, beta2, eps, static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

@@ -53,32 +53,24 @@ struct GatherArgs {
 int gather_rows_launch(const GatherParam* params, int n, const float* buffer, long buffer_len,
                        const int64_t* directions, int ndir, int pairs, hipStream_t s);
 
-struct AdamArgs {
-  float* param;
-  const float* grad;
-  float* m;
-  float* v;
-  long n;
-  float step_size;  // lr / (1 - beta1^step)
-  float beta1, beta2, eps;
-  float bc2_sqrt;   // sqrt(1 - beta2^step)
-};
-
 int fitness_launch(const float* losses, int n, int pairs, int mode, float* fit, float* weight, hipStream_t s);
 int outer_update_launch(const OuterUpdateArgs* mats, int n, const float* w, int ndir, float scale, hipStream_t s);
-int adam_launch(const AdamArgs& g, hipStream_t s);
 
 // Several tensors' Adam steps in one launch: up to ADAM_MAX tensors per launch, passed by value, with the running
-// total of 256-element blocks (block b belongs to the first tensor whose block_end exceeds b).
+// total of ADAM_BLOCK-element blocks (block b belongs to the first tensor whose block_end exceeds b).
 constexpr int ADAM_MAX = 64;
+constexpr int ADAM_BLOCK = 2048;
 struct AdamTensor {
   float* param;
   const float* grad;
   float* m;
   float* v;
   long n;
-  float step_size, bc2_sqrt;
-  long block_end;
+  float step_size;  // lr / (1 - beta1^step)
+  float bc2_sqrt;   // sqrt(1 - beta2^step)
+  // set by the launch
+  int block_end;
+  int vec;          // the four pointers are 16-byte aligned
 };
 struct AdamBatchArgs {
   AdamTensor t[ADAM_MAX];

@@ -184,33 +184,64 @@ __global__ void __launch_bounds__(256) outer_update_kernel(const OuterBatchArgs 
 
 // torch.optim.AdamW (single-tensor path) with weight_decay = 0:
 // m = lerp(m, g, 1 - b1); v = b2 v + (1 - b2) g^2; p -= (lr / bc1) m / (sqrt(v) / sqrt(bc2) + eps).
-__device__ __forceinline__ void adam_element(float* param, const float* grad, float* mp, float* vp, long i,
-                                             float step_size, float bc2_sqrt, float beta1, float beta2, float eps) {
-  const float gr = grad[i];
-  float m = mp[i], v = vp[i];
-  const float w = 1.f - beta1;
-  m = w < 0.5f ? m + w * (gr - m) : gr - (gr - m) * (1.f - w);
-  v = v * beta2 + (1.f - beta2) * gr * gr;
-  mp[i] = m;
-  vp[i] = v;
-  const float denom = sqrtf(v) / bc2_sqrt + eps;
-  param[i] = param[i] + (-step_size) * (m / denom);
+struct AdamConst {
+  float step_size, bc2_sqrt, beta1, beta2, eps;
+};
+__device__ __forceinline__ void adam_element(float& param, float gr, float& m, float& v, const AdamConst& c) {
+  // the fused operations are written out, so that the vector and the scalar path round alike
+  const float w = 1.f - c.beta1, d = gr - m;
+  m = w < 0.5f ? fmaf(w, d, m) : fmaf(-(1.f - w), d, gr);
+  v = fmaf(gr, (1.f - c.beta2) * gr, c.beta2 * v);
+  const float denom = sqrtf(v) / c.bc2_sqrt + c.eps;
+  param = fmaf(-c.step_size, m / denom, param);
 }
-__global__ void __launch_bounds__(256) adam_kernel(AdamArgs g) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= g.n) return;
-  adam_element(g.param, g.grad, g.m, g.v, i, g.step_size, g.bc2_sqrt, g.beta1, g.beta2, g.eps);
-}
-// Every tensor of an optimizer step in one launch (the same arithmetic per element as adam_kernel): block b
-// serves the tensor whose range of 256-element blocks holds it (a uniform scan over the running totals).
+// Every tensor of an optimizer step in one launch: block b serves the tensor whose range of ADAM_BLOCK-element blocks
+// holds it (a binary search over the running totals). Bound by HBM, 28 bytes per element. Four elements per thread and
+// access where the tensor's four pointers allow 16-byte vectors, two of them in flight before any is used: 37.7M
+// parameters 497 us (2.1 TB/s) with one element per thread -> 176 us
+// (6.0 TB/s).
 __global__ void __launch_bounds__(256) adam_batch_kernel(const AdamBatchArgs g) {
   const long b = blockIdx.x;
-  int k = 0;
-  while (k + 1 < g.n && b >= g.t[k].block_end) ++k;
-  const AdamTensor& t = g.t[k];
-  const long i = (b - (k ? g.t[k - 1].block_end : 0)) * 256 + threadIdx.x;
-  if (i >= t.n) return;
-  adam_element(t.param, t.grad, t.m, t.v, i, t.step_size, t.bc2_sqrt, g.beta1, g.beta2, g.eps);
+  int lo = 0, hi = g.n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (b < g.t[mid].block_end) hi = mid;
+    else lo = mid + 1;
+  }
+  const AdamTensor& t = g.t[lo];
+  const AdamConst c{t.step_size, t.bc2_sqrt, g.beta1, g.beta2, g.eps};
+  const long base = (b - (lo ? g.t[lo - 1].block_end : 0)) * ADAM_BLOCK;
+  if (t.vec && base + ADAM_BLOCK <= t.n) {
+    constexpr int V = ADAM_BLOCK / 1024;
+    float4 p4[V], g4[V], m4[V], v4[V];
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      const long i = base + 1024 * q + 4 * threadIdx.x;
+      p4[q] = *reinterpret_cast<const float4*>(t.param + i);
+      g4[q] = *reinterpret_cast<const float4*>(t.grad + i);
+      m4[q] = *reinterpret_cast<const float4*>(t.m + i);
+      v4[q] = *reinterpret_cast<const float4*>(t.v + i);
+    }
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+      const long i = base + 1024 * q + 4 * threadIdx.x;
+      adam_element(p4[q].x, g4[q].x, m4[q].x, v4[q].x, c);
+      adam_element(p4[q].y, g4[q].y, m4[q].y, v4[q].y, c);
+      adam_element(p4[q].z, g4[q].z, m4[q].z, v4[q].z, c);
+      adam_element(p4[q].w, g4[q].w, m4[q].w, v4[q].w, c);
+      *reinterpret_cast<float4*>(t.param + i) = p4[q];
+      *reinterpret_cast<float4*>(t.m + i) = m4[q];
+      *reinterpret_cast<float4*>(t.v + i) = v4[q];
+    }
+    return;
+  }
+  for (long i = base + threadIdx.x; i < min(base + ADAM_BLOCK, t.n); i += 256) {
+    float p = t.param[i], m = t.m[i], v = t.v[i];
+    adam_element(p, t.grad[i], m, v, c);
+    t.param[i] = p;
+    t.m[i] = m;
+    t.v[i] = v;
+  }
 }
 
 }  // namespace
@@ -304,7 +335,7 @@ int adam_batch_launch(const AdamTensor* tensors, int n, float beta1, float beta2
     for (int k = base; k < std::min(n, base + ADAM_MAX); ++k) {
       const AdamTensor& t = tensors[k];
       if (!t.param || !t.grad || !t.m || !t.v || t.n <= 0 || !(t.bc2_sqrt > 0.f)) return NOISE_EINVAL;
-      blocks += (t.n + 255) / 256;
+      blocks += (t.n + ADAM_BLOCK - 1) / ADAM_BLOCK;
     }
     if (blocks > 0x7fffffffL) return NOISE_ENOTSUP;
   }
@@ -314,19 +345,13 @@ int adam_batch_launch(const AdamTensor* tensors, int n, float beta1, float beta2
     g.beta1 = beta1, g.beta2 = beta2, g.eps = eps;
     long blocks = 0;
     for (int k = 0; k < g.n; ++k) {
-      g.t[k] = tensors[base + k];
-      blocks += (g.t[k].n + 255) / 256;
-      g.t[k].block_end = blocks;
+      AdamTensor& t = g.t[k] = tensors[base + k];
+      t.vec = !(((uintptr_t)t.param | (uintptr_t)t.grad | (uintptr_t)t.m | (uintptr_t)t.v) & 15);
+      blocks += (t.n + ADAM_BLOCK - 1) / ADAM_BLOCK;
+      t.block_end = (int)blocks;
     }
     hipLaunchKernelGGL(adam_batch_kernel, dim3((unsigned)blocks), dim3(256), 0, s, g);
     NOISE_CHECK_LAUNCH();
   }
-  return NOISE_OK;
-}
-
-int adam_launch(const AdamArgs& g, hipStream_t s) {
-  if (!g.param || !g.grad || !g.m || !g.v || g.n <= 0 || !(g.bc2_sqrt > 0.f)) return NOISE_EINVAL;
-  hipLaunchKernelGGL(adam_kernel, dim3((unsigned)((g.n + 255) / 256)), dim3(256), 0, s, g);
-  NOISE_CHECK_LAUNCH();
   return NOISE_OK;
 }

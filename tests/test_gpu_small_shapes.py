@@ -183,3 +183,27 @@ def test_attention_of_64_and_128_queries_per_workgroup_agree_bit_for_bit(T, wind
         assert torch.equal(alone[0], other[0]) and torch.equal(alone[1], other[1])
     # (the same kernel's numbers against the oracle: test_attention_matches_oracle_and_moments)
     assert torch.isfinite(alone[0].float()).all()
+
+
+def test_adam_vector_and_scalar_elements_agree():
+    """Tensors of whole and ragged blocks, at 16-byte addresses (four elements per access) and one element off (scalar):
+    the same bits, and nothing written past the end."""
+    import math
+    g = torch.Generator().manual_seed(37)
+    for n in (1, 2047, 2048, 2049, 3 * 2048 + 1023):
+        log_case(f'adam n={n}')
+        vals = [torch.randn(n, generator=g), torch.randn(n, generator=g), torch.randn(n, generator=g),
+                torch.rand(n, generator=g)]
+        res = []
+        for off in (0, 1):
+            bufs = [torch.full((n + 9,), 7.0, device=DEV) for _ in vals]
+            for buf, v in zip(bufs, vals):
+                buf[off:off + n] = v.to(DEV)
+            p, gr, m, v = (buf[off:off + n] for buf in bufs)
+            _lib.call('noise_adam', p.data_ptr(), gr.data_ptr(), m.data_ptr(), v.data_ptr(), n, 1e-3, 0.5, 0.95, 1e-8,
+                      math.sqrt(1 - 0.95), _stream())
+            torch.cuda.synchronize()
+            assert all((buf[off + n:] == 7).all() and (buf[:off] == 7).all() for buf in bufs)
+            res.append((p.clone(), m.clone(), v.clone()))
+        for x, y in zip(*res):
+            assert torch.equal(x, y)
