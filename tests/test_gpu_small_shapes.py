@@ -207,3 +207,20 @@ def test_adam_vector_and_scalar_elements_agree():
             res.append((p.clone(), m.clone(), v.clone()))
         for x, y in zip(*res):
             assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize('pairs', [2, 15, 16, 17, 2047, 2049])
+def test_rank_fitness_of_small_populations_with_ties(pairs):
+    """Sixteen threads per pair, around whole workgroups of 16 pairs and whole tiles of 2048: the oracle's centred ranks
+    bit for bit, many of them ties."""
+    from oracle import eggroll as oe
+    g = torch.Generator().manual_seed(38)
+    log_case(f'rank fitness pairs={pairs}')
+    losses = 8 + torch.randint(0, 50, (2 * pairs,), generator=g) / 64
+    fit, weight = torch.empty(pairs, device=DEV), torch.empty(pairs, device=DEV)
+    dl = losses.to(DEV)
+    _lib.call('noise_fitness', dl.data_ptr(), 2 * pairs, pairs, _lib.FITNESS_RANK, fit.data_ptr(), weight.data_ptr(),
+              _stream())
+    torch.cuda.synchronize()
+    ref, _ = oe.rank_fitness(losses, pairs)
+    assert torch.equal(fit.cpu(), ref)
