@@ -121,6 +121,17 @@ int noise_lowrank_mlp(const void* x, long x_ld, long x_mstride, const void* w_fc
  * (out holds 3 n values). */
 int noise_cast_bf16(const float* in, void* out, long n, int split_cols, noise_stream_t stream);
 
+/* Several fp32 weights [rows, cols] rounded to bf16 in one launch, each row-major (NOISE_LAYOUT_ROWS) or in the tile
+ * GEMM's layout (NOISE_LAYOUT_WTILE: rows % 64 == 0, cols % 32 == 0, out 16-byte aligned): noise_cast_bf16, and
+ * noise_weight_tiles after it, for every weight of a step. mats is a host array, read before the call returns. */
+typedef struct noise_cast {
+  const float* in;
+  void* out;
+  int rows, cols;
+  int layout;
+} noise_cast_t;
+int noise_cast_weights(const noise_cast_t* mats, int n, noise_stream_t stream);
+
 /* x0 = norm(W[idx] + s_p a_p[idx] b_p) fp32 [members*T, 512].
  * Replaces `norm(lowrank_embed(p['transformer.wte.weight'], ...))` (train/val/eggroll.py:61-63, :74). */
 int noise_embed_norm(const float* w, long vocab, const float* a, const float* b, const float* sign,

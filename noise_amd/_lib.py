@@ -31,6 +31,7 @@ SIGNATURES = {
     'noise_lowrank_mlp_workspace_size': [I, I, I, I, SP],
     'noise_lowrank_mlp': [P, L, L, P, P, I, I, P, P, P, P, P, I, I, I, P, P, I, P, S, P],
     'noise_cast_bf16': [P, P, L, I, P],
+    'noise_cast_weights': [P, I, P],
     'noise_embed_norm': [P, L, P, P, P, P, I, I, I, P, P],
     'noise_block_entry': [P, P, P, P, P, P, P, P, P, P, P, P, L, P, P, P, P, P, I, I, I, P, I, P, P],
     'noise_qkv': [P, P, P, P, P, P, P, I, I, I, P, P, P, P, L, P, P, P, L, P, P],
@@ -72,6 +73,18 @@ class OuterMat(ctypes.Structure):
 def outer_mats(items):
     """(a ptr or 0, a_ld, b ptr, b_ld, out, in, grad ptr) tuples -> (pointer to a host array, count)."""
     arr = (OuterMat * len(items))(*[OuterMat(*it) for it in items])
+    return ctypes.cast(arr, P), len(items), arr
+
+
+class Cast(ctypes.Structure):
+    """noise_cast_t of include/noise_hip.h."""
+    _fields_ = [('in', P), ('out', P), ('rows', I), ('cols', I), ('layout', I)]
+
+
+def casts(items):
+    """A host array of noise_cast_t from (in ptr, out ptr, rows, cols, layout) tuples: returns (pointer, count, array) --
+    keep the array alive until the call is enqueued."""
+    arr = (Cast * len(items))(*[Cast(*it) for it in items])
     return ctypes.cast(arr, P), len(items), arr
 
 

@@ -199,6 +199,17 @@ int noise_cast_bf16(const float* in, void* out, long n, int split_cols, noise_st
   return cast_launch(in, static_cast<bf16*>(out), n, split_cols, split_cols > 0, static_cast<hipStream_t>(stream));
 }
 
+int noise_cast_weights(const noise_cast_t* mats, int n, noise_stream_t stream) {
+  if (n <= 0 || !mats) return NOISE_EINVAL;
+  std::vector<CastMat> m(n);
+  for (int k = 0; k < n; ++k) {
+    if (mats[k].layout != NOISE_LAYOUT_ROWS && mats[k].layout != NOISE_LAYOUT_WTILE) return NOISE_EINVAL;
+    m[k] = CastMat{mats[k].in, static_cast<bf16*>(mats[k].out), (long)mats[k].rows * mats[k].cols, mats[k].cols,
+                   mats[k].layout == NOISE_LAYOUT_WTILE};
+  }
+  return cast_batch_launch(m.data(), n, static_cast<hipStream_t>(stream));
+}
+
 int noise_embed_norm(const float* w, long vocab, const float* a, const float* b, const float* sign,
                      const int64_t* idx, int members, int T, int pair_shift, float* x0, noise_stream_t stream) {
   if (bad_members(members, T, pair_shift)) return NOISE_EINVAL;

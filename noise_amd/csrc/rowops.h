@@ -115,6 +115,22 @@ int norm_dot_launch(const NormDotArgs& g, hipStream_t s);
 int head_norm_launch(const HeadNormArgs& g, hipStream_t s);
 int ce_finalize_launch(const CeFinalizeArgs& g, hipStream_t s);
 int cast_launch(const float* in, __bf16* out, long n, int cols, int split, hipStream_t s);
+// Several fp32 matrices rounded to bf16 in one launch, each row-major or in the tile GEMM's WTILE layout (rows % 64 == 0,
+// cols % 32 == 0): up to CAST_MAX per launch, passed by value, with the running total of CAST_BLOCK-element blocks.
+constexpr int CAST_MAX = 64, CAST_BLOCK = 4096;
+struct CastMat {
+  const float* in;
+  __bf16* out;
+  long n;          // rows * cols
+  int cols, tiled;
+  // set by the launch
+  int block_end, vec;
+};
+struct CastBatchArgs {
+  CastMat m[CAST_MAX];
+  int n;
+};
+int cast_batch_launch(const CastMat* mats, int n, hipStream_t s);
 // Row dots u[row] = bf16(sum_k x[row, k] * bf16(b[dir, k])) for a bf16 activation.
 int rowdot_launch(const __bf16* x, long ldx, long x_mstride, int M, int K, int T, int pair_shift,
                   const float* b, long ldb, float* u, hipStream_t stream);

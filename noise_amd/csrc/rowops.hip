@@ -475,6 +475,44 @@ __global__ void __launch_bounds__(256) cast_kernel(const float* __restrict__ in,
   o[2 * cols] = hi;
 }
 
+// Weights of a step in the GEMMs' formats: workgroup b serves the matrix whose range of CAST_BLOCK-element blocks holds
+// it (binary search), each thread 16-byte output chunks of 8 elements. Bound by HBM, 6 bytes per element; one launch for
+// the 48 matrices of the model where a cast per matrix and a WTILE copy per c_proj were 64 launches of 2-4 us (181 us for
+// 25.2M weights, 5.5 us of host time each -> 24.6).
+__global__ void __launch_bounds__(256) cast_batch_kernel(const CastBatchArgs g) {
+  const int b = blockIdx.x;
+  int lo = 0, hi = g.n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (b < g.m[mid].block_end) hi = mid;
+    else lo = mid + 1;
+  }
+  const CastMat& m = g.m[lo];
+  const long c0 = (long)(b - (lo ? g.m[lo - 1].block_end : 0)) * (CAST_BLOCK / 8) + threadIdx.x;
+#pragma unroll
+  for (int i = 0; i < CAST_BLOCK / 8 / 256; ++i) {
+    const long q = c0 + 256 * i;  // output chunk
+    if (8 * q >= m.n) return;
+    long src = 8 * q;
+    if (m.tiled) {
+      // chunk q % 64 of WTILE block q / 64 (wtile_offset's inverse, as in weight_tiles_kernel)
+      const long blk = q >> 6, kt = m.cols >> 5, gb = blk / kt, st = blk - gb * kt;
+      const int u = (int)(q & 63), r = u >> 2, c = (u & 3) ^ ((r >> 1) & 3);
+      const long j = 16 * gb + r;
+      const long n = (j & ~63L) + (r >> 2) * 16 + ((j & 63) >> 4) * 4 + (r & 3);
+      src = n * m.cols + 32 * st + 8 * c;
+    }
+    if (m.vec && 8 * q + 8 <= m.n) {
+      const Row8 v = load8(m.in + src);
+      *reinterpret_cast<uint4*>(m.out + 8 * q) =
+          make_uint4(pack_bf16x2(v.v[0], v.v[1]), pack_bf16x2(v.v[2], v.v[3]), pack_bf16x2(v.v[4], v.v[5]),
+                     pack_bf16x2(v.v[6], v.v[7]));
+    } else {
+      for (int e = 0; e < 8 && 8 * q + e < m.n; ++e) m.out[8 * q + e] = to_bf16(m.in[src + e]);
+    }
+  }
+}
+
 int grid_rows(long M) { return (int)((M + 3) / 4); }
 
 // HBM calibration: one wave per row reads in_kib KiB of the row's source and writes out_kib KiB, with the row
@@ -604,6 +642,32 @@ int cast_launch(const float* in, bf16* out, long n, int cols, int split, hipStre
   if (!in || !out || n <= 0 || (split && (cols <= 0 || n % cols))) return NOISE_EINVAL;
   hipLaunchKernelGGL(cast_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, in, out, n, cols, split);
   NOISE_CHECK_LAUNCH();
+  return NOISE_OK;
+}
+
+int cast_batch_launch(const CastMat* mats, int n, hipStream_t s) {
+  if (n <= 0 || !mats) return NOISE_EINVAL;
+  // every matrix is checked before the first launch: a rejected call writes nothing
+  for (int k = 0; k < n; ++k) {
+    const CastMat& m = mats[k];
+    if (!m.in || !m.out || m.n <= 0 || m.cols <= 0 || m.n % m.cols ||
+        (m.tiled && (m.cols % 32 || m.n / m.cols % 64 || ((uintptr_t)m.out & 15))))
+      return NOISE_EINVAL;
+    if (m.n > (long)CAST_BLOCK * (0x7fffffff / CAST_MAX)) return NOISE_ENOTSUP;
+  }
+  for (int base = 0; base < n; base += CAST_MAX) {
+    CastBatchArgs g{};
+    g.n = n - base < CAST_MAX ? n - base : CAST_MAX;
+    int blocks = 0;
+    for (int k = 0; k < g.n; ++k) {
+      CastMat& m = g.m[k] = mats[base + k];
+      m.vec = !(((uintptr_t)m.in | (uintptr_t)m.out) & 15);
+      blocks += (int)((m.n + CAST_BLOCK - 1) / CAST_BLOCK);
+      m.block_end = blocks;
+    }
+    hipLaunchKernelGGL(cast_batch_kernel, dim3((unsigned)blocks), dim3(256), 0, s, g);
+    NOISE_CHECK_LAUNCH();
+  }
   return NOISE_OK;
 }
 

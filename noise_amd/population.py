@@ -55,16 +55,16 @@ class Weights:
         self.proj = torch.empty(L, D, D, device=dev, dtype=torch.bfloat16)
         self.fc = torch.empty(L, F, D, device=dev, dtype=torch.bfloat16)
         self.mproj = torch.empty(L, D, F, device=dev, dtype=torch.bfloat16)
-        # the MLP c_proj weight (K = 2048, the tile GEMM's operand) is kept in the library's WTILE layout
-        rows = torch.empty(D, F, device=dev, dtype=torch.bfloat16)
+        # every cast of the step in one launch; the MLP c_proj weight (K = 2048, the tile GEMM's operand) is kept in
+        # the library's WTILE layout
+        items = []
         for i in range(L):
             pre = f'transformer.h.{i}.'
             for k, name in enumerate(('attn.c_q.weight', 'attn.c_k.weight', 'attn.c_v.weight')):
-                self._cast(p[pre + name], self.qkv[i, k * D:(k + 1) * D], s)
-            self._cast(p[pre + 'attn.c_proj.weight'], self.proj[i], s)
-            self._cast(p[pre + 'mlp.c_fc.weight'], self.fc[i], s)
-            self._cast(p[pre + 'mlp.c_proj.weight'], rows, s)
-            _lib.call('noise_weight_tiles', rows.data_ptr(), D, F, self.mproj[i].data_ptr(), s)
+                items.append(self._item(p[pre + name], self.qkv, (i * 3 + k) * D * D, (D, D)))
+            items.append(self._item(p[pre + 'attn.c_proj.weight'], self.proj, i * D * D, (D, D)))
+            items.append(self._item(p[pre + 'mlp.c_fc.weight'], self.fc, i * F * D, (F, D)))
+            items.append(self._item(p[pre + 'mlp.c_proj.weight'], self.mproj, i * D * F, (D, F), _lib.LAYOUT_WTILE))
         w_head = p['lm_head.weight']
         V = w_head.shape[0]
         if head == 'fp32':
@@ -76,14 +76,17 @@ class Weights:
             _lib.call('noise_cast_bf16', w_head.data_ptr(), self.head_w.data_ptr(), w_head.numel(), D, s)
         else:
             self.head_w = torch.empty(V, D, device=dev, dtype=torch.bfloat16)
-            self._cast(w_head, self.head_w, s)
+            items.append(self._item(w_head, self.head_w, 0, (V, D)))
+        ptr, count, _keep = _lib.casts(items)
+        _lib.call('noise_cast_weights', ptr, count, s)
 
     @staticmethod
-    def _cast(src, dst, s):
+    def _item(src, dst, at, shape, layout=_lib.LAYOUT_ROWS):
+        """The cast of `src` into the elements of `dst` from `at` on."""
         _need_cuda(src, torch.float32, 'weight')
-        if src.shape != dst.shape:
-            raise ValueError(f'weight shape {tuple(src.shape)} != {tuple(dst.shape)}')
-        _lib.call('noise_cast_bf16', src.data_ptr(), dst.data_ptr(), src.numel(), 0, s)
+        if src.shape != shape:
+            raise ValueError(f'weight shape {tuple(src.shape)} != {shape}')
+        return src.data_ptr(), dst.data_ptr() + 2 * at, *shape, layout
 
 
 class Buffers:

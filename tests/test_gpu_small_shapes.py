@@ -224,3 +224,26 @@ def test_rank_fitness_of_small_populations_with_ties(pairs):
     torch.cuda.synchronize()
     ref, _ = oe.rank_fitness(losses, pairs)
     assert torch.equal(fit.cpu(), ref)
+
+
+@pytest.mark.parametrize('off', [0, 1])
+def test_batched_weight_casts_equal_the_single_ones(off):
+    """noise_cast_weights over more matrices than one launch holds, ragged sizes, both layouts, aligned and misaligned
+    sources: noise_cast_bf16 and noise_weight_tiles bit for bit, and nothing written past a matrix."""
+    g = torch.Generator().manual_seed(39)
+    shapes = [(64, 32), (512, 2048), (1, 1), (3, 7), (5, 4096), (1, 4097), (128, 96)] + [(2, 9)] * 63
+    log_case(f'batched weight casts, source offset {off}')
+    src = [torch.randn(r * c + 1, generator=g).to(DEV)[off:off + r * c] for r, c in shapes]
+    tiled = [r % 64 == 0 and c % 32 == 0 for r, c in shapes]
+    out = [torch.full((r * c + 8,), 7., device=DEV, dtype=torch.bfloat16) for r, c in shapes]
+    ptr, n, _keep = _lib.casts([(x.data_ptr(), o.data_ptr(), r, c, _lib.LAYOUT_WTILE if t else _lib.LAYOUT_ROWS)
+                                for x, o, (r, c), t in zip(src, out, shapes, tiled)])
+    _lib.call('noise_cast_weights', ptr, n, _stream())
+    for x, o, (r, c), t in zip(src, out, shapes, tiled):
+        ref = torch.empty(r * c, device=DEV, dtype=torch.bfloat16)
+        _lib.call('noise_cast_bf16', x.data_ptr(), ref.data_ptr(), r * c, 0, _stream())
+        if t:
+            rows, ref = ref, torch.empty_like(ref)
+            _lib.call('noise_weight_tiles', rows.data_ptr(), r, c, ref.data_ptr(), _stream())
+        torch.cuda.synchronize()
+        assert torch.equal(o[:r * c], ref) and (o[r * c:] == 7).all(), (r, c)
