@@ -390,6 +390,88 @@ int noise_gather_rows(const float* buffer, long buffer_len, const noise_gather_p
 int noise_adam(float* param, const float* grad, float* exp_avg, float* exp_avg_sq, long n, float step_size,
                float beta1, float beta2, float eps, float bc2_sqrt, noise_stream_t stream);
 
+/* ---------------------------------------------------------------- whole passes
+ * The stages above in the reference's order, issued by one call: every launch a caller would compose itself, with the
+ * same arguments, so the results are the same bits. All pointers are device memory unless said otherwise; null where the
+ * stage's own entry point takes null. */
+typedef struct noise_forward_layer { /* one block; a_x / b_x: the first perturbation row of the matrix's [dirs, out] / [dirs, in] */
+  const void* w_qkv;   /* bf16 [1536, 512] = c_q ; c_k ; c_v */
+  const void* w_proj;  /* bf16 [512, 512] */
+  const void* w_fc;    /* bf16 [2048, 512] */
+  const void* w_mproj; /* bf16 [512, 2048] in NOISE_LAYOUT_WTILE */
+  const float *a_q, *b_q, *a_k, *b_k, *a_v, *b_v, *a_proj, *b_proj, *a_fc, *b_fc, *a_mproj, *b_mproj;
+  const float *gate_w, *gate_a, *gate_b; /* value gate; null: a block without value embedding */
+  const float *ve_w, *ve_a, *ve_b;
+  int window;
+} noise_forward_layer_t;
+
+/* `population_loss` on one chunk of members (train/val/eggroll.py:66-103). */
+typedef struct noise_forward {
+  const noise_forward_layer_t* layers; /* host array, read before the call returns */
+  int n_layer;
+  const float* wte; /* [vocab, 512], perturbed by wte_a [dirs, vocab], wte_b [dirs, 512] */
+  long vocab;
+  const float *wte_a, *wte_b;
+  const float *lambda_r, *lambda_0, *eps_r, *eps_0; /* per layer; eps rows eps_ld apart */
+  long eps_ld;
+  const void *rot_cos, *rot_sin;
+  const int64_t *idx, *targets;
+  long tok_mstride;
+  const float* sign;
+  int members, T, pair_shift;
+  const void* head_w;
+  int head_vocab, head_format;
+  const float *head_a, *head_b;
+  int reduction;
+  float *loss, *logits;
+  /* buffers of members * T rows */
+  float* x;     /* [512] */
+  void* h;      /* bf16 [512] */
+  float* u_qkv; /* [4] */
+  float* gate;  /* [8] */
+  void* qkv;    /* [1536] */
+  void* y;      /* bf16 [512] */
+  float* u_attn; /* [8] */
+  void *y_ap, *y_mp; /* bf16 [512] */
+  float* u_fc;  /* [1] */
+  void* hidden; /* bf16 [2048] */
+  float* u_mlp; /* part-major [u_mlp_parts, rows]: noise_mlp_fc_parts(2048) */
+  int u_mlp_parts;
+  void* head_ws;
+  size_t head_ws_bytes;
+} noise_forward_t;
+/* Stages first .. last - 1 of the pass: 6 i + k for block i (0 block entry, 1 q | k | v, 2 attention, 3 attention c_proj,
+ * 4 MLP entry, 5 the MLP's two products), 6 n_layer for the head. */
+int noise_forward(const noise_forward_t* f, int first, int last, noise_stream_t stream);
+
+/* GPT.forward under torch's bf16 autocast (utils/eval.py:44-45), from the noise_ac_* stages: batch sequences of T tokens
+ * (token stride T). Of the layers, only the weights, gate_w, ve_w and window are read. */
+typedef struct noise_autocast {
+  const noise_forward_layer_t* layers; /* host array */
+  int n_layer;
+  const float* wte;
+  long vocab;
+  const float *lambda_r, *lambda_0;
+  const void *rot_cos, *rot_sin;
+  const int64_t *idx, *targets;
+  int batch, T;
+  const void* head_w; /* bf16 [head_vocab, 512] */
+  int head_vocab, reduction;
+  float *loss, *logits;
+  const float* zeros; /* max(batch * 2048, batch * head_vocab, batch * T) floats of value 0 */
+  void *x, *h, *xf, *y, *y_ap, *y_mp; /* bf16 rows of 512 */
+  void *qkv, *hidden; /* bf16 rows of 1536 and 2048 */
+  float *gate, *upart;
+  void* head_ws;
+  size_t head_ws_bytes;
+} noise_autocast_t;
+int noise_autocast_forward(const noise_autocast_t* f, noise_stream_t stream);
+
+/* Smallest and largest of na token ids a and nb ids b (either count may be 0): out [NOISE_TOKEN_RANGE_PARTS, 4] partial
+ * {min a, max a, min b, max b} (INT64_MAX / INT64_MIN where a part saw none), every one written. */
+#define NOISE_TOKEN_RANGE_PARTS 32
+int noise_token_range(const int64_t* a, long na, const int64_t* b, long nb, int64_t* out, noise_stream_t stream);
+
 /* HBM streaming calibration (no counterpart in the reference): each of `rows` rows reads in_kib KiB of src and writes
  * out_kib KiB of dst (1..4 KiB each, 16-byte aligned buffers), one wave per row with the row kernels' 16-byte vector
  * accesses. It measures the bandwidth ceiling of a row kernel's read / write mix (bench.py --workload stream). */

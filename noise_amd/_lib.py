@@ -49,6 +49,9 @@ SIGNATURES = {
     'noise_mlp_fc': [P, P, I, I, P, P, P, P, I, I, I, P, I, P, P],
     'noise_head_ce_workspace_size': [I, I, I, I, SP],
     'noise_head_ce': [P, I, P, P, I, I, P, P, P, P, L, I, I, I, I, P, P, P, S, P, I, P],
+    'noise_forward': [P, I, I, P],
+    'noise_autocast_forward': [P, P],
+    'noise_token_range': [P, L, P, L, P, P],
     'noise_fitness': [P, I, I, I, P, P, P],
     'noise_outer_update': [P, L, P, L, P, I, I, I, F, P, P],
     'noise_outer_update_batch': [P, I, P, I, F, P],
@@ -86,6 +89,36 @@ def casts(items):
     keep the array alive until the call is enqueued."""
     arr = (Cast * len(items))(*[Cast(*it) for it in items])
     return ctypes.cast(arr, P), len(items), arr
+
+
+class ForwardLayer(ctypes.Structure):
+    """noise_forward_layer_t of include/noise_hip.h."""
+    _fields_ = [(n, P) for n in ('w_qkv', 'w_proj', 'w_fc', 'w_mproj', 'a_q', 'b_q', 'a_k', 'b_k', 'a_v', 'b_v', 'a_proj',
+                                 'b_proj', 'a_fc', 'b_fc', 'a_mproj', 'b_mproj', 'gate_w', 'gate_a', 'gate_b', 've_w',
+                                 've_a', 've_b')] + [('window', I)]
+
+
+class Forward(ctypes.Structure):
+    """noise_forward_t of include/noise_hip.h."""
+    _fields_ = [('layers', ctypes.POINTER(ForwardLayer)), ('n_layer', I), ('wte', P), ('vocab', L), ('wte_a', P),
+                ('wte_b', P), ('lambda_r', P), ('lambda_0', P), ('eps_r', P), ('eps_0', P), ('eps_ld', L), ('rot_cos', P),
+                ('rot_sin', P), ('idx', P), ('targets', P), ('tok_mstride', L), ('sign', P), ('members', I), ('T', I),
+                ('pair_shift', I), ('head_w', P), ('head_vocab', I), ('head_format', I), ('head_a', P), ('head_b', P),
+                ('reduction', I), ('loss', P), ('logits', P), ('x', P), ('h', P), ('u_qkv', P), ('gate', P), ('qkv', P),
+                ('y', P), ('u_attn', P), ('y_ap', P), ('y_mp', P), ('u_fc', P), ('hidden', P), ('u_mlp', P),
+                ('u_mlp_parts', I), ('head_ws', P), ('head_ws_bytes', S)]
+
+
+class Autocast(ctypes.Structure):
+    """noise_autocast_t of include/noise_hip.h."""
+    _fields_ = [('layers', ctypes.POINTER(ForwardLayer)), ('n_layer', I), ('wte', P), ('vocab', L), ('lambda_r', P),
+                ('lambda_0', P), ('rot_cos', P), ('rot_sin', P), ('idx', P), ('targets', P), ('batch', I), ('T', I),
+                ('head_w', P), ('head_vocab', I), ('reduction', I), ('loss', P), ('logits', P), ('zeros', P), ('x', P),
+                ('h', P), ('xf', P), ('y', P), ('y_ap', P), ('y_mp', P), ('qkv', P), ('hidden', P), ('gate', P),
+                ('upart', P), ('head_ws', P), ('head_ws_bytes', S)]
+
+
+TOKEN_RANGE_PARTS = 32
 
 
 class GatherParam(ctypes.Structure):

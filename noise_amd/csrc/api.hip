@@ -561,6 +561,10 @@ int noise_head_ce(const void* x, int x_bf16, const float* gain, const void* w_he
   return ce_finalize_launch(f, s);
 }
 
+int noise_token_range(const int64_t* a, long na, const int64_t* b, long nb, int64_t* out, noise_stream_t stream) {
+  return token_range_launch(a, na, b, nb, out, NOISE_TOKEN_RANGE_PARTS, static_cast<hipStream_t>(stream));
+}
+
 int noise_fitness(const float* losses, int n, int pairs, int mode, float* fitness, float* weight,
                   noise_stream_t stream) {
   return fitness_launch(losses, n, pairs, mode, fitness, weight, static_cast<hipStream_t>(stream));

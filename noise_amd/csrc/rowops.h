@@ -113,6 +113,8 @@ int hbm_stream_launch(const void* src, int in_kib, void* dst, int out_kib, long 
 int block_entry_launch(const BlockEntryArgs& g, hipStream_t s);
 int norm_dot_launch(const NormDotArgs& g, hipStream_t s);
 int head_norm_launch(const HeadNormArgs& g, hipStream_t s);
+// Partial {min a, max a, min b, max b} of two token id arrays: out [parts, 4].
+int token_range_launch(const int64_t* a, long na, const int64_t* b, long nb, int64_t* out, int parts, hipStream_t s);
 int ce_finalize_launch(const CeFinalizeArgs& g, hipStream_t s);
 int cast_launch(const float* in, __bf16* out, long n, int cols, int split, hipStream_t s);
 // Several fp32 matrices rounded to bf16 in one launch, each row-major or in the tile GEMM's WTILE layout (rows % 64 == 0,

@@ -513,6 +513,33 @@ __global__ void __launch_bounds__(256) cast_batch_kernel(const CastBatchArgs g) 
   }
 }
 
+// Workgroup k of `parts` scans every parts-th 256-element run of both arrays and writes its partial.
+__global__ void __launch_bounds__(256) token_range_kernel(const int64_t* __restrict__ a, long na,
+                                                          const int64_t* __restrict__ b, long nb,
+                                                          int64_t* __restrict__ out) {
+  __shared__ int64_t red[4][4];
+  int64_t v[4] = {INT64_MAX, INT64_MIN, INT64_MAX, INT64_MIN};
+  const long step = (long)gridDim.x * 256, i0 = (long)blockIdx.x * 256 + threadIdx.x;
+  for (long i = i0; i < na; i += step) v[0] = min(v[0], a[i]), v[1] = max(v[1], a[i]);
+  for (long i = i0; i < nb; i += step) v[2] = min(v[2], b[i]), v[3] = max(v[3], b[i]);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+      const int64_t w = __shfl_xor((long long)v[k], o);
+      v[k] = (k & 1) ? max(v[k], w) : min(v[k], w);
+    }
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = v[k];
+  }
+  __syncthreads();
+  if (threadIdx.x < 4) {
+    const int k = threadIdx.x;
+    int64_t r = red[0][k];
+    for (int w = 1; w < 4; ++w) r = (k & 1) ? max(r, red[w][k]) : min(r, red[w][k]);
+    out[4 * blockIdx.x + k] = r;
+  }
+}
+
 int grid_rows(long M) { return (int)((M + 3) / 4); }
 
 // HBM calibration: one wave per row reads in_kib KiB of the row's source and writes out_kib KiB, with the row
@@ -641,6 +668,13 @@ int ce_finalize_launch(const CeFinalizeArgs& g, hipStream_t s) {
 int cast_launch(const float* in, bf16* out, long n, int cols, int split, hipStream_t s) {
   if (!in || !out || n <= 0 || (split && (cols <= 0 || n % cols))) return NOISE_EINVAL;
   hipLaunchKernelGGL(cast_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, in, out, n, cols, split);
+  NOISE_CHECK_LAUNCH();
+  return NOISE_OK;
+}
+
+int token_range_launch(const int64_t* a, long na, const int64_t* b, long nb, int64_t* out, int parts, hipStream_t s) {
+  if (na < 0 || nb < 0 || na + nb == 0 || (na && !a) || (nb && !b) || !out || parts <= 0) return NOISE_EINVAL;
+  hipLaunchKernelGGL(token_range_kernel, dim3((unsigned)parts), dim3(256), 0, s, a, na, b, nb, out);
   NOISE_CHECK_LAUNCH();
   return NOISE_OK;
 }

@@ -6,6 +6,8 @@ forward runs in libnoise_hip.so. Members are evaluated in chunks so activations 
 of m members at T tokens holds about m * T * 13 KiB of activations (fp32 residual stream, bf16 q|k|v,
 attention output and the 2048-wide MLP hidden; x0 is recomputed, never stored).
 """
+import ctypes
+
 import torch
 
 from . import _lib
@@ -117,14 +119,6 @@ class Buffers:
         return members <= self.members and T == self.T
 
 
-def _noise_rows(noise, name, lo, hi):
-    """Rows lo..hi of a (a, b) pair or of an eps matrix, as contiguous device tensors."""
-    n = noise[name]
-    if isinstance(n, tuple):
-        return tuple(t[lo:hi] for t in n)
-    return n[lo:hi]
-
-
 class StageTimer:
     """Optional per-stage timing of forward_chunk: HIP events recorded on the launch stream around each
     stage (embed, entry, qkv, attention, attn_proj, mlp, head); `ms` accumulates milliseconds per
@@ -166,14 +160,40 @@ class _NoTimer:
 TIMER = _NoTimer()
 
 
-# q and k reach attention RMS-normalised (noise_qkv applies the QK-norm), so its bounded-score softmax applies
-QK_NORM = True
+# the stages of noise_forward: six per block, then the head
+BLOCK_STAGES = ('entry', 'qkv', 'attention', 'attn_proj', 'mlp_entry', 'mlp')
+
+
+def _layers(W, p, cfg, windows, rows):
+    """The blocks' weights (GEMM operands of W, value gates and embeddings of p), and the perturbation rows that
+    `rows(name)` -> (a, b) pointers gives (None: no perturbation)."""
+    out = (_lib.ForwardLayer * cfg.n_layer)()
+    qkv, proj, fc, mproj = (t.data_ptr() for t in (W.qkv, W.proj, W.fc, W.mproj))
+    none = (None, None)
+    for i, lay in enumerate(out):
+        lay.w_qkv, lay.w_proj = qkv + 6 * D * D * i, proj + 2 * D * D * i
+        lay.w_fc, lay.w_mproj = fc + 2 * F * D * i, mproj + 2 * F * D * i
+        lay.window = windows[i]
+        pre = f'transformer.h.{i}.'
+        if has_ve(i, cfg.n_layer):
+            lay.gate_w, lay.ve_w = p[pre + 'attn.ve_gate.weight'].data_ptr(), p[f'value_embeds.{i}.weight'].data_ptr()
+            lay.gate_a, lay.gate_b = rows(pre + 'attn.ve_gate.weight') if rows else none
+            lay.ve_a, lay.ve_b = rows(f'value_embeds.{i}.weight') if rows else none
+        if rows:
+            lay.a_q, lay.b_q = rows(pre + 'attn.c_q.weight')
+            lay.a_k, lay.b_k = rows(pre + 'attn.c_k.weight')
+            lay.a_v, lay.b_v = rows(pre + 'attn.c_v.weight')
+            lay.a_proj, lay.b_proj = rows(pre + 'attn.c_proj.weight')
+            lay.a_fc, lay.b_fc = rows(pre + 'mlp.c_fc.weight')
+            lay.a_mproj, lay.b_mproj = rows(pre + 'mlp.c_proj.weight')
+    return out
 
 
 def forward_chunk(W, buf, noise, sign, idx, targets, pair_shift, out, cos, sin, windows, tok_mstride=0,
-                  reduction=_lib.CE_MEMBER_MEAN, logits=None):
+                  reduction=_lib.CE_MEMBER_MEAN, logits=None, row0=0):
     """Losses of members 0..m-1 of `sign` (m = len(sign)) into `out` (per member, or reduced as
-    `reduction` says); noise rows are indexed by p >> pair_shift. Member p reads the token ids and targets
+    `reduction` says); noise rows are indexed by row0 + (p >> pair_shift); `noise` is the perturbation dict, or one
+    tensor of zeros that every matrix's rows fit in. Member p reads the token ids and targets
     at p * tok_mstride (0: one shared sequence). When `logits` is given, the capped logits are written there
     too (targets and out may then be None). Follows train/val/eggroll.py:72-103 op for op."""
     tm = TIMER
@@ -193,80 +213,52 @@ def forward_chunk(W, buf, noise, sign, idx, targets, pair_shift, out, cos, sin, 
         nout = m * T if reduction == _lib.CE_NONE else m if reduction == _lib.CE_MEMBER_MEAN else 1
         if out.numel() < nout:
             raise ValueError(f'out must hold {nout} losses')
-    s = _stream()
-    ps = pair_shift
-    a, b = noise['transformer.wte.weight']
-    V = p['transformer.wte.weight'].shape[0]
-    # x0 = norm(lowrank_embed(wte)) (train/val/eggroll.py:74) is never stored: every block entry recomputes its
-    # rows from the L2-resident table (the same arithmetic as noise_embed_norm), which saves reading a 4 KiB
-    # per member-token fp32 stream from HBM at each of the n_layer blocks
-    emb, emb_ptr = _lib.embed(_p(p['transformer.wte.weight']), V, _p(a), _p(b), _p(idx), tok_mstride)
-    eps_r, eps_0 = noise['resid_lambdas'], noise['x0_lambdas']
-    lam_r, lam_0 = p['resid_lambdas'], p['x0_lambdas']
-    # Deferred residuals. `x = x + lowrank(c_proj, ...)` (train/val/eggroll.py:92-93) is split: the c_proj GEMM
-    # writes only its bf16 dense product, and the next kernel that reads the residual stream adds the rank-1
-    # term and the residual with the same fp32 operations, in the same order (the MLP entry for the attention
-    # output; the next block entry, or the head, for both outputs of a block).
-    pend_prev = []
-    for i in range(cfg.n_layer):
-        pre = f'transformer.h.{i}.'
-        aq, bq = noise[pre + 'attn.c_q.weight']
-        ak, bk = noise[pre + 'attn.c_k.weight']
-        av, bv = noise[pre + 'attn.c_v.weight']
-        ve = has_ve(i, cfg.n_layer)
-        if ve:
-            gw = p[pre + 'attn.ve_gate.weight']
-            ga, gb = noise[pre + 'attn.ve_gate.weight']
-            vw = p[f'value_embeds.{i}.weight']
-            va, vb = noise[f'value_embeds.{i}.weight']
-        x_in = None if i == 0 else _p(buf.x)
-        t0 = tm.mark('entry')
-        pend, npend = _lib.pending(*pend_prev)
-        _lib.call('noise_block_entry', x_in, None, _p(buf.x), _p(buf.h), _p(buf.u_qkv), _p(bq), _p(bk),
-                  _p(bv), lam_r.data_ptr() + 4 * i, lam_0.data_ptr() + 4 * i, eps_r.data_ptr() + 4 * i,
-                  eps_0.data_ptr() + 4 * i, eps_r.stride(0), _p(gw) if ve else 0, _p(ga) if ve else 0,
-                  _p(gb) if ve else 0, _p(buf.gate) if ve else 0, _p(sign), m, T, ps, pend, npend, emb_ptr, s)
+    if isinstance(noise, torch.Tensor):
+        zero = noise.data_ptr()
+        eps_r = eps_0 = zero
+        eps_ld = cfg.n_layer
+
+        def rows(name):
+            return zero, zero
+    else:
+        nr, n0 = noise['resid_lambdas'], noise['x0_lambdas']
+        eps_ld = nr.stride(0)
+        eps_r, eps_0 = nr.data_ptr() + 4 * row0 * eps_ld, n0.data_ptr() + 4 * row0 * eps_ld
+
+        def rows(name):
+            a, b = noise[name]
+            return a.data_ptr() + 4 * row0 * a.shape[1], b.data_ptr() + 4 * row0 * b.shape[1]
+    wte = p['transformer.wte.weight']
+    f = _lib.Forward(_layers(W, p, cfg, windows, rows), cfg.n_layer, wte.data_ptr(), wte.shape[0],
+                     *rows('transformer.wte.weight'), p['resid_lambdas'].data_ptr(), p['x0_lambdas'].data_ptr(), eps_r,
+                     eps_0, eps_ld, cos.data_ptr(), sin.data_ptr(), _p(idx), _p(targets), tok_mstride, sign.data_ptr(), m,
+                     T, pair_shift, W.head_w.data_ptr(), W.head_w.shape[0], HEAD_FORMAT[W.head],
+                     *rows('lm_head.weight'), reduction, _p(out), _p(logits),
+                     *(t.data_ptr() for t in (buf.x, buf.h, buf.u_qkv, buf.gate, buf.qkv, buf.y, buf.u_attn, buf.y_ap,
+                                              buf.y_mp, buf.u_fc, buf.hidden, buf.u_mlp)),
+                     buf.parts, buf.head_ws.data_ptr(), buf.head_ws.numel())
+    s, n = _stream(), len(BLOCK_STAGES) * cfg.n_layer
+    if isinstance(tm, _NoTimer):
+        _lib.call('noise_forward', ctypes.byref(f), 0, n + 1, s)
+        return
+    for k in range(n + 1):
+        t0 = tm.mark(BLOCK_STAGES[k % len(BLOCK_STAGES)] if k < n else 'head')
+        _lib.call('noise_forward', ctypes.byref(f), k, k + 1, s)
         tm.close(t0)
-        t0 = tm.mark('qkv')
-        _lib.call('noise_qkv', _p(buf.h), _p(W.qkv[i]), _p(aq), _p(ak), _p(av), _p(buf.u_qkv), _p(sign), m, T, ps,
-                  _p(cos), _p(sin), _p(buf.gate) if ve else 0, _p(vw) if ve else 0, V, _p(va) if ve else 0,
-                  _p(vb) if ve else 0, _p(idx), tok_mstride, _p(buf.qkv), s)
-        tm.close(t0)
-        ap, bp = noise[pre + 'attn.c_proj.weight']
-        t0 = tm.mark('attention')
-        # q and k come out of noise_qkv RMS-normalised
-        _lib.call('noise_attention', _p(buf.qkv), m, T, windows[i], int(QK_NORM), _lib.QK_F16_Q_LOG2, _p(bp), ps,
-                  _p(buf.y), _p(buf.u_attn), 0, 0, 0, s)
-        tm.close(t0)
-        t0 = tm.mark('attn_proj')
-        _lib.call('noise_dense_bf16', _p(buf.y), _lib.LAYOUT_ROWS, D, D, _p(W.proj[i]), _lib.LAYOUT_ROWS, m, T,
-                  _p(buf.y_ap), s)
-        tm.close(t0)
-        attn_out = (_p(buf.y_ap), _p(buf.u_attn), H, H, 1, _p(ap))
-        af, bf_ = noise[pre + 'mlp.c_fc.weight']
-        am, bm = noise[pre + 'mlp.c_proj.weight']
-        t0 = tm.mark('mlp_entry')
-        pend, npend = _lib.pending(attn_out)
-        _lib.call('noise_norm_dot', _p(buf.x), _p(buf.h), _p(bf_), _p(buf.u_fc), _p(sign), m, T, ps, pend, npend, s)
-        tm.close(t0)
-        t0 = tm.mark('mlp')
-        # the hidden stays in the library's TILE16 layout between the two MLP GEMMs
-        _lib.call('noise_mlp_fc', _p(buf.h), _p(W.fc[i]), D, F, _p(af), _p(buf.u_fc), _p(bm), _p(sign), m, T, ps,
-                  _p(buf.hidden), _lib.LAYOUT_TILE16, _p(buf.u_mlp), s)
-        _lib.call('noise_dense_bf16', _p(buf.hidden), _lib.LAYOUT_TILE16, F, D, _p(W.mproj[i]), _lib.LAYOUT_WTILE, m,
-                  T, _p(buf.y_mp), s)
-        tm.close(t0)
-        # the fc partials are part-major with stride m * T (this chunk's rows)
-        mlp_out = (_p(buf.y_mp), _p(buf.u_mlp), buf.parts, 1, m * T, _p(am))
-        pend_prev = [attn_out, mlp_out]
-    ah, bh = noise['lm_head.weight']
-    Vh = W.head_w.shape[0]
-    t0 = tm.mark('head')
-    pend, npend = _lib.pending(*pend_prev)
-    _lib.call('noise_head_ce', _p(buf.x), 0, 0, _p(W.head_w), Vh, HEAD_FORMAT[W.head], _p(ah), _p(bh), _p(sign),
-              _p(targets), tok_mstride, m, T, ps, reduction, _p(out), _p(logits), _p(buf.head_ws), buf.head_ws.numel(),
-              pend, npend, s)
-    tm.close(t0)
+
+
+def token_range(a, b=None):
+    """Launches the search for the extremes of one or two int64 id tensors (one kernel); the returned function waits for
+    it and gives (min a, max a) or (min a, max a, min b, max b). A caller reads it after its other launches and host work
+    and before the kernels that index by the ids."""
+    part = torch.empty(_lib.TOKEN_RANGE_PARTS, 4, device=a.device, dtype=torch.int64)
+    _lib.call('noise_token_range', a.data_ptr(), a.numel(), _p(b), 0 if b is None else b.numel(), part.data_ptr(),
+              _stream())
+
+    def read():
+        lo_a, hi_a, lo_b, hi_b = zip(*part.tolist())
+        return (min(lo_a), max(hi_a)) + (() if b is None else (min(lo_b), max(hi_b)))
+    return read
 
 
 def check_noise(noise, shapes, rows):
@@ -274,6 +266,9 @@ def check_noise(noise, shapes, rows):
         n = noise[name]
         if len(shape) == 2:
             a, b = n
+            if a.is_cuda and b.is_cuda and a.dtype == b.dtype == torch.float32 and a.is_contiguous() and \
+                    b.is_contiguous() and len(a) >= rows and len(b) >= rows and (a.shape[1], b.shape[1]) == shape:
+                continue
             _need_cuda(a, torch.float32, f'noise[{name}][0]')
             _need_cuda(b, torch.float32, f'noise[{name}][1]')
             if a.shape[0] < rows or b.shape[0] < rows or a.shape[1] != shape[0] or b.shape[1] != shape[1]:
@@ -330,10 +325,7 @@ class Population:
         if T % 128:
             raise ValueError(f'T = {T} must be a multiple of 128 (attention query blocks)')
         V = p['transformer.wte.weight'].shape[0]
-        lo = torch.minimum(idx.min(), targets.min()).item()
-        hi = torch.maximum(idx.max(), targets.max()).item()
-        if lo < 0 or hi >= V:
-            raise IndexError(f'token ids must lie in [0, {V}), got [{lo}, {hi}]')
+        ids = token_range(idx, targets)
         rows = (m + (1 << pair_shift) - 1) >> pair_shift
         check_noise(noise, {n: tuple(t.shape) for n, t in p.items()}, rows)
         W = weights or Weights(p, self.config, self.head)
@@ -341,13 +333,15 @@ class Population:
         out = torch.empty(m, device=dev, dtype=torch.float32)
         step = self.chunk if pair_shift == 0 else self.chunk - self.chunk % 2
         buf = self.buffers(min(step, m), T, dev)
+        lo_i, hi_i, lo_t, hi_t = ids()
+        lo, hi = min(lo_i, lo_t), max(hi_i, hi_t)
+        if lo < 0 or hi >= V:
+            raise IndexError(f'token ids must lie in [0, {V}), got [{lo}, {hi}]')
         for c0 in range(0, m, step):
             c1 = min(m, c0 + step)
-            r0, r1 = c0 >> pair_shift, (c1 + (1 << pair_shift) - 1) >> pair_shift
-            chunk_noise = {n: _noise_rows(noise, n, r0, r1) for n in p}
             ci, ct = (idx[c0:c1], targets[c0:c1]) if per_member else (idx, targets)
-            forward_chunk(W, buf, chunk_noise, sign[c0:c1], ci, ct, pair_shift, out[c0:c1], cos, sin,
-                          self.windows, tok_mstride=T if per_member else 0)
+            forward_chunk(W, buf, noise, sign[c0:c1], ci, ct, pair_shift, out[c0:c1], cos, sin, self.windows,
+                          tok_mstride=T if per_member else 0, row0=c0 >> pair_shift)
         return out
 
 
@@ -371,16 +365,19 @@ def _check_clean_inputs(model, idx, targets, loss_reduction):
     if T % 128:
         raise ValueError(f'T = {T} must be a multiple of 128 (attention query blocks)')
     V = model.transformer.wte.weight.shape[0]
-    if idx.min().item() < 0 or idx.max().item() >= V:
-        raise IndexError(f'token ids must lie in [0, {V})')
     if targets is not None:
         _need_cuda(targets, torch.int64, 'targets')
         if targets.shape != idx.shape:
             raise ValueError(f'targets must be {tuple(idx.shape)}, got {tuple(targets.shape)}')
-        valid = targets != -1
-        if ((targets < 0) & valid).any().item() or (targets >= V).any().item():
+    ids = token_range(idx, targets)
+
+    def check():
+        r = ids()
+        if r[0] < 0 or r[1] >= V:
+            raise IndexError(f'token ids must lie in [0, {V})')
+        if targets is not None and (r[2] < -1 or r[3] >= V):
             raise IndexError(f'targets must lie in [0, {V}) or be -1 (ignored)')
-    return B, T, V
+    return B, T, V, check
 
 
 def autocast_forward(model, idx, targets=None, loss_reduction='mean', weights=None):
@@ -392,65 +389,41 @@ def autocast_forward(model, idx, targets=None, loss_reduction='mean', weights=No
     q, k, v with bf16 probabilities, noise_mlp_fc at sigma = 0 (relu(bf16)^2 rounded to bf16 where c_proj casts it)
     and the bf16 head with the fp32 cap and cross-entropy (noise_head_ce). Same returns as clean_forward. The
     embedding tables are read as bf16 (fp32 tensors holding bf16 values, as noise_amd.eval.load_model keeps them)."""
-    B, T, V = _check_clean_inputs(model, idx, targets, loss_reduction)
+    B, T, V, check_ids = _check_clean_inputs(model, idx, targets, loss_reduction)
     cfg = model.config
     p = dict(model.named_parameters())
     dev = idx.device
     W = weights or Weights(p, cfg, 'bf16')
     if W.head != 'bf16':
         raise ValueError("the autocast forward needs bf16 head weights (Weights(p, config, 'bf16'))")
-    s = _stream()
     M = B * T
     b16 = torch.bfloat16
-    x, h, xf = (torch.empty(M, D, device=dev, dtype=b16) for _ in range(3))
-    y, y_ap, y_mp = (torch.empty(M, D, device=dev, dtype=b16) for _ in range(3))
-    qkv = torch.empty(M, 3 * D, device=dev, dtype=b16)
-    hidden = torch.empty(M, F, device=dev, dtype=b16)
-    gate = torch.empty(M, H, device=dev)
-    parts = _lib.value('noise_mlp_fc_parts', F)
-    upart = torch.empty(parts, M, device=dev)
+    Vh = W.head_w.shape[0]
+    x, h, xf, y, y_ap, y_mp = (torch.empty(M, D, device=dev, dtype=b16) for _ in range(6))
+    qkv, hidden = torch.empty(M, 3 * D, device=dev, dtype=b16), torch.empty(M, F, device=dev, dtype=b16)
+    gate, upart = torch.empty(M, H, device=dev), torch.empty(_lib.value('noise_mlp_fc_parts', F), M, device=dev)
     # sigma = 0: zero rank-1 vectors and signs, so noise_mlp_fc and the head add exactly nothing
-    zf, zb, zu, zsign = (torch.zeros(B, F, device=dev), torch.zeros(B, F, device=dev), torch.zeros(M, device=dev),
-                         torch.zeros(B, device=dev))
-    za, zbh = torch.zeros(B, W.head_w.shape[0], device=dev), torch.zeros(B, D, device=dev)
+    zeros = torch.zeros(B * max(F, Vh, T), device=dev)
     pop = Population(model, chunk=B, head='bf16')
     cos, sin = pop.tables(T)
     idx = idx.contiguous()
-    wte = p['transformer.wte.weight']
-    lam_r, lam_0 = p['resid_lambdas'], p['x0_lambdas']
-    for i in range(cfg.n_layer):
-        pre = f'transformer.h.{i}.'
-        ve = has_ve(i, cfg.n_layer)
-        first = i == 0
-        _lib.call('noise_ac_stream', None if first else _p(x), _p(wte), V, _p(idx), T, None if first else _p(y_ap),
-                  None if first else _p(y_mp), lam_r.data_ptr() + 4 * i, lam_0.data_ptr() + 4 * i, _p(x), _p(h),
-                  _p(p[pre + 'attn.ve_gate.weight']) if ve else None, _p(gate) if ve else None, M, T, s)
-        _lib.call('noise_dense_bf16', _p(h), _lib.LAYOUT_ROWS, D, 3 * D, _p(W.qkv[i]), _lib.LAYOUT_ROWS, B, T, _p(qkv), s)
-        vw = p[f'value_embeds.{i}.weight'] if ve else None
-        _lib.call('noise_ac_qkv', _p(qkv), _p(cos), _p(sin), _p(gate) if ve else None, _p(vw), V if ve else 0,
-                  _p(idx), T, M, T, s)
-        _lib.call('noise_attention', _p(qkv), B, T, pop.windows[i], 1, _lib.QK_BF16_V_BF16, None, 0, _p(y), None, None,
-                  None, 0, s)
-        _lib.call('noise_dense_bf16', _p(y), _lib.LAYOUT_ROWS, D, D, _p(W.proj[i]), _lib.LAYOUT_ROWS, B, T, _p(y_ap), s)
-        _lib.call('noise_ac_stream', _p(x), None, 0, None, 0, _p(y_ap), None, None, None, None, _p(h), None, None, M, T,
-                  s)
-        _lib.call('noise_mlp_fc', _p(h), _p(W.fc[i]), D, F, _p(zf), _p(zu), _p(zb), _p(zsign), B, T, 0, _p(hidden),
-                  _lib.LAYOUT_TILE16, _p(upart), s)
-        _lib.call('noise_dense_bf16', _p(hidden), _lib.LAYOUT_TILE16, F, D, _p(W.mproj[i]), _lib.LAYOUT_WTILE, B, T,
-                  _p(y_mp), s)
-    _lib.call('noise_ac_stream', _p(x), None, 0, None, 0, _p(y_ap), _p(y_mp), None, None, _p(xf), None, None, None, M, T,
-              s)
-    Vh = W.head_w.shape[0]
+    targets = None if targets is None else targets.contiguous()
     ws = torch.empty(_lib.size_query('noise_head_ce_workspace_size', B, T, Vh, 0), device=dev, dtype=torch.uint8)
+    red, out, logits = _lib.CE_MEMBER_MEAN, None, None
     if targets is None:
         logits = torch.empty(B, T, Vh, device=dev)
-        _lib.call('noise_head_ce', _p(xf), 1, None, _p(W.head_w), Vh, 0, _p(za), _p(zbh), _p(zsign), None, T, B, T, 0,
-                  _lib.CE_MEMBER_MEAN, None, _p(logits), _p(ws), ws.numel(), None, 0, s)
+    else:
+        red = REDUCTIONS[loss_reduction]
+        out = torch.empty(M if red == _lib.CE_NONE else 1, device=dev)
+    wte = p['transformer.wte.weight']
+    f = _lib.Autocast(_layers(W, p, cfg, pop.windows, None), cfg.n_layer, wte.data_ptr(), V, p['resid_lambdas'].data_ptr(),
+                      p['x0_lambdas'].data_ptr(), cos.data_ptr(), sin.data_ptr(), idx.data_ptr(), _p(targets), B, T,
+                      W.head_w.data_ptr(), Vh, red, _p(out), _p(logits),
+                      *(t.data_ptr() for t in (zeros, x, h, xf, y, y_ap, y_mp, qkv, hidden, gate, upart, ws)), ws.numel())
+    check_ids()
+    _lib.call('noise_autocast_forward', ctypes.byref(f), _stream())
+    if targets is None:
         return logits
-    red = REDUCTIONS[loss_reduction]
-    out = torch.empty(M if red == _lib.CE_NONE else 1, device=dev)
-    _lib.call('noise_head_ce', _p(xf), 1, None, _p(W.head_w), Vh, 0, _p(za), _p(zbh), _p(zsign),
-              _p(targets.contiguous()), T, B, T, 0, red, _p(out), None, _p(ws), ws.numel(), None, 0, s)
     return out if red == _lib.CE_NONE else out[0]
 
 
@@ -464,12 +437,11 @@ def clean_forward(model, idx, targets=None, loss_reduction='mean', head='fp32', 
     fp32 logits [B, T, vocab] are returned. The kernels keep the rounding points of the population path (fp32
     residual stream and norms, bf16 GEMMs, fp16 attention operands), not the all-bf16 stream GPT.forward has under
     autocast with bf16 embeddings; head='fp32' keeps the head fp32-accurate, 'bf16' rounds it as autocast does."""
-    B, T, V = _check_clean_inputs(model, idx, targets, loss_reduction)
+    B, T, V, check_ids = _check_clean_inputs(model, idx, targets, loss_reduction)
     p = dict(model.named_parameters())
     dev = idx.device
-    # sigma = 0: zero signs and zero noise rows (finite, so s * (x . b) * a is exactly zero)
-    noise = {n: (torch.zeros(B, t.shape[0], device=dev), torch.zeros(B, t.shape[1], device=dev)) if t.dim() == 2
-             else torch.zeros(B, t.shape[0], device=dev) for n, t in p.items()}
+    # sigma = 0: zero signs and zero noise rows (finite, so s * (x . b) * a is exactly zero), one buffer for all of them
+    noise = torch.zeros(B, max(n for t in p.values() for n in t.shape), device=dev)
     sign = torch.zeros(B, device=dev)
     pop = Population(model, chunk=B, head=head)
     W = weights or Weights(p, model.config, head)
@@ -477,9 +449,11 @@ def clean_forward(model, idx, targets=None, loss_reduction='mean', head='fp32', 
     buf = pop.buffers(B, T, dev)
     if targets is None:
         logits = torch.empty(B, T, W.head_w.shape[0], device=dev, dtype=torch.float32)
+        check_ids()
         forward_chunk(W, buf, noise, sign, idx, None, 0, None, cos, sin, pop.windows, tok_mstride=T, logits=logits)
         return logits
     red = REDUCTIONS[loss_reduction]
     out = torch.empty(B * T if red == _lib.CE_NONE else 1, device=dev, dtype=torch.float32)
+    check_ids()
     forward_chunk(W, buf, noise, sign, idx, targets, 0, out, cos, sin, pop.windows, tok_mstride=T, reduction=red)
     return out if red == _lib.CE_NONE else out[0]

@@ -247,3 +247,43 @@ def test_batched_weight_casts_equal_the_single_ones(off):
             _lib.call('noise_weight_tiles', rows.data_ptr(), r, c, ref.data_ptr(), _stream())
         torch.cuda.synchronize()
         assert torch.equal(o[:r * c], ref) and (o[r * c:] == 7).all(), (r, c)
+
+
+@pytest.mark.parametrize('na,nb', [(1, 0), (5, 300), (8192, 8192), (8193, 1), (100003, 7)])
+def test_token_range(na, nb):
+    """The id check's partials over fewer ids than one workgroup, exactly the launch, and past it: the exact extremes."""
+    from noise_amd.population import token_range
+    g = torch.Generator().manual_seed(40)
+    log_case(f'token_range {na} {nb}')
+    a = torch.randint(-2 ** 62, 2 ** 62, (na,), generator=g)
+    b = torch.randint(-2 ** 62, 2 ** 62, (nb,), generator=g) if nb else None
+    want = (int(a.min()), int(a.max())) + ((int(b.min()), int(b.max())) if nb else ())
+    assert token_range(a.to(DEV), None if b is None else b.to(DEV))() == want
+
+
+def test_forward_stage_by_stage_equals_the_whole_pass():
+    """noise_forward one stage at a time (as a stage timer drives it), in chunks whose noise rows start past 0, and in one
+    call: the same losses bit for bit."""
+    from noise_amd import population
+    from noise_amd.model import make_model
+    from noise_amd.synthetic import antithetic_signs, population_noise, trained_like, zipf_tokens
+    m, T = 6, 128
+    log_case('forward stage by stage')
+    model = trained_like(make_model('cpu', 0)).to(DEV)
+    p = dict(model.named_parameters())
+    noise = {n: tuple(t.to(DEV) for t in v) if isinstance(v, tuple) else v.to(DEV)
+             for n, v in population_noise({n: tuple(t.shape) for n, t in p.items()}, m // 2, per_member=False).items()}
+    idx, tgt = (t.to(DEV) for t in zipf_tokens(T))
+    sign = antithetic_signs(m, 1e-2).to(DEV)
+
+    def loss(chunk):
+        return population.Population(model, chunk=chunk).loss(p, noise, sign, idx, tgt, pair_shift=1)
+    whole = loss(m)
+    assert torch.equal(loss(2), whole) and torch.equal(loss(4), whole)
+    population.TIMER = timer = population.StageTimer()
+    try:
+        assert torch.equal(loss(m), whole)
+    finally:
+        population.TIMER = population._NoTimer()
+    timer.collect()
+    assert timer.count == {**{s: 8 for s in population.BLOCK_STAGES}, 'head': 1}
