@@ -287,3 +287,79 @@ def test_forward_stage_by_stage_equals_the_whole_pass():
         population.TIMER = population._NoTimer()
     timer.collect()
     assert timer.count == {**{s: 8 for s in population.BLOCK_STAGES}, 'head': 1}
+
+
+def _outer_case(g, shapes, n):
+    mats = []
+    for o, i, pad in shapes:
+        a = torch.randn(n, o + pad, generator=g)[:, :o] if o else None
+        mats.append((a, torch.randn(n, i + pad, generator=g)[:, :i]))
+    return mats, torch.randn(n, generator=g)
+
+
+def _outer_gpu(mats, w, scale):
+    dev = [(None if a is None else _strided(a), _strided(b)) for a, b in mats]
+    grads = [torch.full((max(1, 0 if a is None else a.shape[1]) * b.shape[1] + 4,), 7., device=DEV) for a, b in mats]
+    wd = w.to(DEV)
+    ptr, cnt, _keep = _lib.outer_mats([(0 if a is None else a.data_ptr(), 0 if a is None else a.stride(0), b.data_ptr(),
+                                        b.stride(0), 1 if a is None else a.shape[1], b.shape[1], gr.data_ptr())
+                                       for (a, b), gr in zip(dev, grads)])
+    _lib.call('noise_outer_update_batch', ptr, cnt, wd.data_ptr(), len(w), scale, _stream())
+    torch.cuda.synchronize()
+    out = []
+    for (a, b), gr in zip(mats, grads):
+        assert (gr[-4:] == 7).all()  # nothing past the matrix
+        out.append(gr[:-4].view(-1, b.shape[1]).cpu())
+    return out
+
+
+def _strided(t):
+    """t on the GPU with the row stride it has on the host."""
+    buf = torch.zeros(t.shape[0], t.stride(0), device=DEV)
+    buf[:, :t.shape[1]] = t.to(DEV)
+    return buf[:, :t.shape[1]]
+
+
+@pytest.mark.parametrize('n', [1, 31, 33, 100])
+def test_outer_update_on_split_operands(n):
+    """Enough 128 x 128 tiles for the bf16-split kernel (288 of them in one matrix), ragged outputs, padded and odd row
+    strides, a vector parameter, direction counts around its 32-direction chunks: against the fp64 sum. The split drops
+    terms below 2^-24 of a product and rounds 6 times per 32 directions (2^-23 allows for truncation inside an MFMA), and
+    w a is rounded once."""
+    g = torch.Generator().manual_seed(41)
+    log_case(f'outer update, split operands, {n} directions')
+    mats, w = _outer_case(g, [(4100, 1000, 0), (130, 257, 3), (0, 8, 0), (8, 32, 1), (1, 1, 0), (128, 128, 4)], n)
+    for (a, b), got in zip(mats, _outer_gpu(mats, w, -0.25)):
+        wa = (torch.ones(n, 1) if a is None else a).double() * w.double()[:, None]
+        ref, mag = wa.t() @ b.double() * -0.25, wa.abs().t() @ b.double().abs() * 0.25
+        bound = (4 + 6 * (n // 32 + 1)) * 2 ** -23 * mag
+        assert ((got.double() - ref).abs() <= bound).all()
+
+
+def test_outer_update_of_non_finite_and_extreme_values():
+    """Infinities, NaN and values that bf16 would round to infinity: what the fp32 sum gives, in that column or row only;
+    tiny values (a product of 1e-30) keep their sum."""
+    g = torch.Generator().manual_seed(42)
+    n = 40
+    log_case('outer update of non-finite and extreme values')
+    mats, w = _outer_case(g, [(4100, 1000, 0)], n)
+    a, b = mats[0]
+    w = w.abs() + 0.5
+    w[3] = 1
+    b[3] = b[3].abs() + 0.1  # (no infinity times zero, and infinities of one sign per row)
+    a[3, 5], a[3, 6], a[7, 2000], b[9, 700] = float('inf'), float('-inf'), float('nan'), float('inf')
+    a[9] = a[9].abs() + 0.1
+    a[:, 17], a[3, 17] = 0, 3.4e38  # past bf16's largest; with b[3, 1] = 2^-100 finite
+    b[3, 1] = 2 ** -100
+    a[:, 4000] *= 1e-30
+    got = _outer_gpu(mats, w, 1.0)[0]
+    ref = torch.zeros(4100, 1000)
+    for j in range(n):
+        ref += (w[j] * a[j])[:, None] * b[j][None]
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    inf = torch.isinf(ref)
+    assert torch.equal(torch.isinf(got), inf) and torch.equal(got[inf], ref[inf])
+    ok = torch.isfinite(ref)
+    mag = (w[:, None].double() * a.double()).abs().nan_to_num(0, 0, 0).t() @ b.double().abs().nan_to_num(0, 0, 0)
+    assert ((got.double() - ref.double()).abs()[ok] <= ((4 + 6 * 2 + n) * 2 ** -23 * mag)[ok]).all()
+    assert (got[4000, :700] != 0).all()
