@@ -202,8 +202,10 @@ lowrank_gemm_kernel(const LowrankGemmArgs g) {
     // The dense product issues its loads from inline assembly, which the compiler's wait insertion does not see:
     // with the builtin it waits vmcnt(0) before the next LDS read at a tile's first and last steps (measured: MLP
     // pair 23.83 -> 23.62 ms). The loop's own waits (open) order every stage read after its loads. The other
-    // epilogues keep the builtin: their M0 saves and restores cost more than the waits (config 3 13.27 -> 13.75 ms).
-    if constexpr (EPI == EPI_DENSE) {
+    // epilogues keep the builtin in the large tiles: their M0 saves and restores cost more than the waits (config 3
+    // 13.27 -> 13.75 ms); in the 64 x 64 ones (FM = 1) the waits cost more (with the steady loop, 64 rows: the fp32 head
+    // 28.1 -> 21.7 us, the split one 35.7 -> 25.7, the linear at K = 2048 16.7 -> 14.9).
+    if constexpr (EPI == EPI_DENSE || FM == 1) {
 #pragma unroll
       for (int d = 0; d < C::LA; ++d) dma_x4(g.A + a_src[d] + ka, sx + (wave * C::LA + d) * 512);
 #pragma unroll
@@ -312,9 +314,9 @@ lowrank_gemm_kernel(const LowrankGemmArgs g) {
   };
   constexpr std::true_type steady{};
   constexpr std::false_type general{};
-  // the dense product and the head run their steady steps from a loop of their own; the other epilogues keep
-  // one loop (with a second one, config 1's EPI_STORE product measured 4% slower)
-  constexpr bool STEADY_LOOP = SUB == 1 && (EPI == EPI_DENSE || CE);
+  // the dense product, the head and the 64 x 64 tiles run their steady steps from a loop of their own; the other
+  // epilogues keep one loop (with a second one, config 1's EPI_STORE product measured 4% slower)
+  constexpr bool STEADY_LOOP = SUB == 1 && (EPI == EPI_DENSE || CE || FM == 1);
   // Step t's MFMAs with (wc, xf) while step t + 1's operands are read into (wn_, xf).
   auto step_read = [&](int t, const bf16x8 (&wc)[FN], bf16x8 (&wn_)[FN], auto st) {
     open(t + 1, st);
