@@ -99,7 +99,8 @@ enum : int {
 };
 struct CeFinalizeArgs {
   const float* part;     // [members * T, parts] sums of exp(z)
-  const float* tgt;      // [members * T] z at the target (written only where the target is valid)
+  float* tgt;            // [members * T] z at the target (written only where the target is valid); the sums overwrite it
+                         // with the rows' losses
   int parts, members, T;
   float* loss;           // [members] / [members * T] / [1] by reduction
   const int64_t* targets;  // member p, position t: targets[p * tgt_mstride + t]

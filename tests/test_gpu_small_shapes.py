@@ -363,3 +363,46 @@ def test_outer_update_of_non_finite_and_extreme_values():
     mag = (w[:, None].double() * a.double()).abs().nan_to_num(0, 0, 0).t() @ b.double().abs().nan_to_num(0, 0, 0)
     assert ((got.double() - ref.double()).abs()[ok] <= ((4 + 6 * 2 + n) * 2 ** -23 * mag)[ok]).all()
     assert (got[4000, :700] != 0).all()
+
+
+@pytest.mark.parametrize('members,T', [(1, 5), (3, 16), (2, 4096), (1, 8230), (5, 130)])
+def test_loss_reductions_add_the_row_losses_in_their_fixed_order(members, T):
+    """Member means, sum and mean of the head's losses, rows below one chain step, around whole LDS tiles of 4096 and past
+    them, some targets ignored: bit for bit the sixteen strided fp32 chains of the per-row losses, added in order."""
+    g = torch.Generator().manual_seed(43)
+    V, M = 256, members * T
+    log_case(f'loss reductions members={members} T={T}')
+    x, w = torch.randn(M, 512, generator=g).to(DEV), (torch.randn(V, 512, generator=g) * 0.05).to(DEV)
+    a, b, sign = torch.zeros(members, V, device=DEV), torch.zeros(members, 512, device=DEV), torch.zeros(members, device=DEV)
+    tgt = torch.randint(0, V, (M,), generator=g)
+    n = _lib.size_query('noise_head_ce_workspace_size', members, T, V, _lib.HEAD_FP32)
+    ws = torch.empty(n, device=DEV, dtype=torch.uint8)
+
+    def run(red, targets, size):
+        t, loss = targets.to(DEV), torch.empty(size, device=DEV)
+        _lib.call('noise_head_ce', x.data_ptr(), 0, None, w.data_ptr(), V, _lib.HEAD_FP32, a.data_ptr(), b.data_ptr(),
+                  sign.data_ptr(), t.data_ptr(), T, members, T, 0, red, loss.data_ptr(), None, ws.data_ptr(), n, None, 0,
+                  _stream())
+        torch.cuda.synchronize()
+        return loss.cpu()
+
+    def chains(rows, valid):
+        acc = torch.zeros(16)
+        for i in range(0, len(rows), 16):
+            k = min(16, len(rows) - i)
+            acc[:k] = torch.where(valid[i:i + k], acc[:k] + rows[i:i + k], acc[:k])
+        t = torch.zeros(())
+        for v in acc:
+            t = t + v
+        return t
+    rows = run(_lib.CE_NONE, tgt, M)
+    every = torch.ones(T, dtype=torch.bool)
+    means = torch.stack([chains(rows[p * T:(p + 1) * T], every) / torch.tensor(float(T)) for p in range(members)])
+    assert torch.equal(run(_lib.CE_MEMBER_MEAN, tgt, members), means)
+    tgt[::3] = -1
+    valid, rows = tgt != -1, run(_lib.CE_NONE, tgt, M)
+    total = chains(rows, valid)
+    assert torch.equal(run(_lib.CE_SUM, tgt, 1)[0], total)
+    assert torch.equal(run(_lib.CE_MEAN, tgt, 1)[0], total / valid.sum().float())
+    if M > 16:
+        assert torch.isnan(run(_lib.CE_MEAN, torch.full((M,), -1), 1)).all()
