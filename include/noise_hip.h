@@ -222,9 +222,12 @@ int noise_attention_noalloc(const void* qkv, int members, int T, int window, int
  * q, k and v are 16-bit rows of 512 (8 heads x 64), 16-byte aligned, in q_blocks, k_blocks and v_blocks consecutive
  * blocks of T rows; member p reads block p % blocks of each, so an operand that members share (the reruns' fixed heads
  * and values: one block per batch row, members ordered draw by draw) is stored once. Each count divides members. No
- * c_proj dots and no moments. */
+ * c_proj dots and no moments. When score is not null, it receives what noise_head_scores makes of y (y itself may then
+ * be null): baseline and target fp32 [score_blocks, T, 8, 64] (16-byte aligned), member j * score_blocks + b being draw j
+ * of batch row b, score [score_blocks, 8, T, draws]. */
 int noise_attention_heads(const void* q, int q_blocks, const void* k, int k_blocks, const void* v, int v_blocks,
-                          int members, int T, int window, int qk_norm, int qk_format, void* y, noise_stream_t stream);
+                          int members, int T, int window, int qk_norm, int qk_format, void* y, const float* baseline,
+                          const float* target, int score_blocks, float* score, noise_stream_t stream);
 
 /* resid += lowrank(x, w) with the input-side dot of row r given as u_parts partial sums
  * u[r * u_row_stride + q * u_part_stride]: the attention c_proj (u from noise_attention: row stride 8,

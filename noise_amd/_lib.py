@@ -38,7 +38,7 @@ SIGNATURES = {
     'noise_attention_workspace_size': [I, I, SP],
     'noise_attention': [P, I, I, I, I, I, P, I, P, P, P, P, S, P],
     'noise_attention_noalloc': [P, I, I, I, I, I, P, I, P, P, P, P],
-    'noise_attention_heads': [P, I, P, I, P, I, I, I, I, I, I, P, P],
+    'noise_attention_heads': [P, I, P, I, P, I, I, I, I, I, I, P, P, P, I, P, P],
     'noise_lowrank_resid': [P, P, I, I, P, P, I, L, L, P, I, I, I, P, P],
     'noise_norm_dot': [P, P, P, P, P, I, I, I, P, I, P],
     'noise_ac_stream': [P, P, L, P, L, P, P, P, P, P, P, P, P, I, I, P],

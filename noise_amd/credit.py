@@ -38,6 +38,12 @@ def _rows(t):
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
+def _f32_rows(t):
+    """t as contiguous fp32 rows at a 16-byte address."""
+    t = t.float().contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _value_rows(t):
     """The bf16-rounded values in fp16, the kernel's operand format."""
     return t.to(torch.bfloat16).to(torch.float16, memory_format=torch.contiguous_format)
@@ -126,16 +132,12 @@ def attention(q, k, v, window, qk_norm=False):
     q, k, v = _rows(q), _rows(k), _value_rows(v)
     y = torch.empty(B * T, H * HD, device=q.device, dtype=torch.bfloat16)
     _lib.call('noise_attention_heads', q.data_ptr(), B, k.data_ptr(), B, v.data_ptr(), B, B, T, int(window),
-              int(bool(qk_norm)), _lib.QK_BF16, y.data_ptr(), _stream())
+              int(bool(qk_norm)), _lib.QK_BF16, y.data_ptr(), None, None, 0, None, _stream())
     return y.view(B, T, H, HD)
 
 
-def rerun(kind, raw, a, sigma, cos, sin, fixed, values, window):
-    """The attention reruns of one chunk of draws in `query_key_errors` (train/val/run.py:618-622): the moved heads of
-    `kind` ('q' or 'k') against the other processed head `fixed` and `values` (both [b, t, h, 64]), which every draw
-    reads from the one copy (64 draws of 2048 tokens: the broadcast copies beside each draw's moved heads took 202 us,
-    and the moved heads' own rows 68 instead of 42). Returns the attention output [n, b, t, h, 64] bf16. Both heads hold
-    RMS-normalised rows, so the kernel runs with bounded scores (no running maximum)."""
+def _rerun(kind, raw, a, sigma, cos, sin, fixed, values, window, scored=None):
+    """rerun's output or, with scored = (baseline, target), the head scores of it."""
     if kind not in ('q', 'k'):
         raise ValueError("kind must be 'q' or 'k'")
     n, b, T, H, hd = a.shape
@@ -149,6 +151,8 @@ def rerun(kind, raw, a, sigma, cos, sin, fixed, values, window):
         raise TypeError('a must be bfloat16')
     if window < 0:
         raise ValueError('window must be >= 0')
+    if scored is not None and not all(tuple(t.shape) == (b, T, H, HD) for t in scored):
+        raise ValueError('baseline and hub must be [b, t, h, 64] like one draw of out')
     cos, sin = _tables(cos, T), _tables(sin, T)
     _cuda(raw, 'raw'), _cuda(a, 'a'), _cuda(fixed, 'fixed'), _cuda(values, 'values')
     W = H * HD
@@ -160,10 +164,32 @@ def rerun(kind, raw, a, sigma, cos, sin, fixed, values, window):
               T, H, moved.data_ptr(), W, stream)
     # every draw reads the same b blocks of fixed heads and values
     q, k = ((moved, n * b), (fixed, b)) if kind == 'q' else ((fixed, b), (moved, n * b))
-    y = torch.empty(n * b * T, W, device=a.device, dtype=torch.bfloat16)
+    if scored is None:
+        out, base, target = torch.empty(n, b, T, H, HD, device=a.device, dtype=torch.bfloat16), None, None
+        y, score = out.data_ptr(), None
+    else:
+        base, target = (_f32_rows(_cuda(t, 'baseline and target')) for t in scored)
+        out = torch.empty(b, H, T, n, device=a.device, dtype=torch.float32)
+        y, score = None, out.data_ptr()
     _lib.call('noise_attention_heads', q[0].data_ptr(), q[1], k[0].data_ptr(), k[1], values.data_ptr(), b, n * b, T,
-              int(window), 1, _lib.QK_BF16, y.data_ptr(), stream)
-    return y.view(n, b, T, H, HD)
+              int(window), 1, _lib.QK_BF16, y, None if base is None else base.data_ptr(),
+              None if target is None else target.data_ptr(), b, score, stream)
+    return out
+
+
+def rerun(kind, raw, a, sigma, cos, sin, fixed, values, window):
+    """The attention reruns of one chunk of draws in `query_key_errors` (train/val/run.py:618-622): the moved heads of
+    `kind` ('q' or 'k') against the other processed head `fixed` and `values` (both [b, t, h, 64]), which every draw
+    reads from the one copy (64 draws of 2048 tokens: the broadcast copies beside each draw's moved heads took 202 us,
+    and the moved heads' own rows 68 instead of 42). Returns the attention output [n, b, t, h, 64] bf16. Both heads hold
+    RMS-normalised rows, so the kernel runs with bounded scores (no running maximum)."""
+    return _rerun(kind, raw, a, sigma, cos, sin, fixed, values, window)
+
+
+def rerun_scores(kind, raw, a, sigma, cos, sin, fixed, values, window, baseline, hub):
+    """head_scores(rerun(...), baseline, hub), [b, h, t, n] fp32, from the attention kernel's epilogue: the outputs are
+    neither written nor read back (64 draws of 2048 tokens: 134 MB each way)."""
+    return _rerun(kind, raw, a, sigma, cos, sin, fixed, values, window, (baseline, hub))
 
 
 def credit_chunk(kind, raw, a, sigma, cos, sin, fixed, values, window, baseline, target, key_filter=None):
@@ -174,8 +200,7 @@ def credit_chunk(kind, raw, a, sigma, cos, sin, fixed, values, window, baseline,
     n, b, T, H, _ = a.shape
     if kind == 'k' and (key_filter is None or tuple(key_filter.shape) != (b, H, T, T)):
         raise ValueError(f'key credit needs the matched filter key_filter [{b}, {H}, {T}, {T}]')
-    out = rerun(kind, raw, a, sigma, cos, sin, fixed, values, window)
-    score = head_scores(out, baseline, target)
+    score = rerun_scores(kind, raw, a, sigma, cos, sin, fixed, values, window, baseline, target)
     if kind == 'k':
         score = key_scores(key_filter, score)
     return code_estimate(score, a)

@@ -356,7 +356,8 @@ int noise_attention_noalloc(const void* qkv, int members, int T, int window, int
 }
 
 int noise_attention_heads(const void* q, int q_blocks, const void* k, int k_blocks, const void* v, int v_blocks,
-                          int members, int T, int window, int qk_norm, int qk_format, void* y, noise_stream_t stream) {
+                          int members, int T, int window, int qk_norm, int qk_format, void* y, const float* baseline,
+                          const float* target, int score_blocks, float* score, noise_stream_t stream) {
   if (bad_members(members, T, 0)) return NOISE_EINVAL;
   for (const int blocks : {q_blocks, k_blocks, v_blocks})
     if (blocks <= 0 || members % blocks) return NOISE_EINVAL;
@@ -372,6 +373,10 @@ int noise_attention_heads(const void* q, int q_blocks, const void* k, int k_bloc
   g.window = window;
   g.qk_norm = qk_norm != 0;
   g.qk_format = qk_format;
+  g.base = baseline;
+  g.target = target;
+  g.score_blocks = score_blocks;
+  g.score = score;
   return attention_launch(g, static_cast<hipStream_t>(stream));
 }
 

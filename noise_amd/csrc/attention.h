@@ -15,7 +15,7 @@ struct AttnHeads {
 };
 struct AttnArgs {
   AttnHeads q, k, v;  // v fp16 (bf16 for QK_BF16_V_BF16)
-  __bf16* y;          // [members * T, ldy], head h at columns h*64 .. h*64+63
+  __bf16* y;          // [members * T, ldy], head h at columns h*64 .. h*64+63; null: only the scores below
   long ldy;
   int members, T, H, window;
   int qk_norm;        // q and k rows are RMS-normalised (scores bounded by 8.03): no running maximum
@@ -31,6 +31,13 @@ struct AttnArgs {
   // mom_out [members, H, 2, 64] (mean of y, mean of y^2); nullable
   float* mom;
   float* mom_out;
+  // scores of the output's change: member p = draw j * score_blocks + block writes, per head and query t,
+  // score[((block * H + h) * T + t) * draws + j] = sum_d (y - base) target over the head's 64 dims, base and target fp32
+  // [score_blocks, T, H, 64]; nullable
+  const float* base;
+  const float* target;
+  float* score;
+  int score_blocks;
 };
 
 // Floats of the moment partials workspace.

@@ -360,10 +360,29 @@ __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) yv[4 * db + e] = bf16r(o[qb][db][e] * inv);
     // ordinary stores: the four lane groups fill 32 bytes of each row per instruction, which L2 merges
-    bf16* out = g.y + row * g.ldy + h * HD + 4 * grp;
+    if (g.y) {
+      bf16* out = g.y + row * g.ldy + h * HD + 4 * grp;
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
-      *reinterpret_cast<uint2*>(out + 16 * db) = make_uint2(pack2(yv[4 * db], yv[4 * db + 1]), pack2(yv[4 * db + 2], yv[4 * db + 3]));
+      for (int db = 0; db < 4; ++db)
+        *reinterpret_cast<uint2*>(out + 16 * db) =
+            make_uint2(pack2(yv[4 * db], yv[4 * db + 1]), pack2(yv[4 * db + 2], yv[4 * db + 3]));
+    }
+    if (g.score) {
+      // the credit reruns' head scores (train/val/run.py:192-195) from the rounded output while it is in registers: the
+      // reruns' outputs are neither written nor read back
+      const int blk = p % g.score_blocks, draw = p / g.score_blocks;
+      const long at = (((long)blk * g.T + q) * g.H + h) * HD + 4 * grp;
+      float d = 0.f;
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+        const float4 b4 = *reinterpret_cast<const float4*>(g.base + at + 16 * db);
+        const float4 t4 = *reinterpret_cast<const float4*>(g.target + at + 16 * db);
+        d += (yv[4 * db] - b4.x) * t4.x + (yv[4 * db + 1] - b4.y) * t4.y + (yv[4 * db + 2] - b4.z) * t4.z +
+             (yv[4 * db + 3] - b4.w) * t4.w;
+      }
+      d = sum_rows4(d);
+      if (grp == 0) g.score[(((long)blk * g.H + h) * g.T + q) * (g.members / g.score_blocks) + draw] = d;
+    }
     if (g.upart) {
       const float* br = g.b_proj + (long)dir * g.b_ld + h * HD + 4 * grp;
       float d = 0.f;
@@ -418,7 +437,7 @@ __global__ void moments_reduce_kernel(const float* part, float* out, int nqb, in
 long attention_moment_partials(int members, int T, int H) { return (long)members * H * (T / BQ_MAX) * 2 * HD; }
 
 int attention_launch(const AttnArgs& g, hipStream_t s) {
-  if (!g.y || g.members <= 0 || g.T <= 0 || g.T % BQ_MAX || g.T % BKV || g.H <= 0 || g.window < 0 || g.ldy % 8 ||
+  if ((!g.y && !g.score) || g.members <= 0 || g.T <= 0 || g.T % BQ_MAX || g.T % BKV || g.H <= 0 || g.window < 0 || g.ldy % 8 ||
       ((uintptr_t)g.y & 15))
     return NOISE_EINVAL;
   for (const AttnHeads* o : {&g.q, &g.k, &g.v})
@@ -427,6 +446,9 @@ int attention_launch(const AttnArgs& g, hipStream_t s) {
       return NOISE_EINVAL;
   if (g.upart && (!g.b_proj || g.upart_ld < g.H || g.b_ld < g.H * HD)) return NOISE_EINVAL;
   if (g.mom && !g.mom_out) return NOISE_EINVAL;
+  if (g.score && (!g.base || !g.target || g.score_blocks <= 0 || g.members % g.score_blocks ||
+                  (((uintptr_t)g.base | (uintptr_t)g.target) & 15)))
+    return NOISE_EINVAL;
   if (g.qk_format < QK_BF16 || g.qk_format > QK_BF16_V_BF16 ||
       ((g.qk_format == QK_F16_Q_LOG2 || g.qk_format == QK_BF16_V_BF16) && !g.qk_norm))
     return NOISE_EINVAL;

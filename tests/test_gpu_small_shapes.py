@@ -121,7 +121,7 @@ def test_attention_on_shared_heads_equals_packed_rows(shared, qk_norm):
     q, k = ((fixed, b), (own, n * b)) if shared == 'q' else ((own, n * b), (fixed, b))
     y = torch.empty(n * b * T, 512, device=DEV, dtype=torch.bfloat16)
     _lib.call('noise_attention_heads', q[0].data_ptr(), q[1], k[0].data_ptr(), k[1], v.data_ptr(), b, n * b, T, window,
-              qk_norm, _lib.QK_BF16, y.data_ptr(), _stream())
+              qk_norm, _lib.QK_BF16, y.data_ptr(), None, None, 0, None, _stream())
     rows = torch.cat([t[0].repeat(n * b // t[1], 1) for t in (q, k, (v.view(torch.bfloat16), b))], 1).contiguous()
     ref = torch.empty_like(y)
     _lib.call('noise_attention', rows.data_ptr(), n * b, T, window, qk_norm, _lib.QK_BF16, None, 0, ref.data_ptr(), None,
@@ -406,3 +406,29 @@ def test_loss_reductions_add_the_row_losses_in_their_fixed_order(members, T):
     assert torch.equal(run(_lib.CE_MEAN, tgt, 1)[0], total / valid.sum().float())
     if M > 16:
         assert torch.isnan(run(_lib.CE_MEAN, torch.full((M,), -1), 1)).all()
+
+
+@pytest.mark.parametrize('kind', ['q', 'k'])
+@pytest.mark.parametrize('n,b,T,window', [(3, 2, 128, 40), (70, 1, 256, 300), (9, 2, 1152, 1100)])
+def test_scores_of_a_credit_chunk_equal_those_of_its_outputs(kind, n, b, T, window):
+    """The attention epilogue's head scores (outputs never written) against noise_head_scores on the outputs of the same
+    reruns, with fp32 and bf16, strided and misaligned baselines: the same 64 fp32 products added in another order, 64
+    2^-23 of their magnitudes. Small grids (64 queries per workgroup) and ones that fill the GPU."""
+    from noise_amd import credit
+    g = torch.Generator(DEV).manual_seed(45)
+    log_case(f'scores of a credit chunk {kind} n={n} b={b} T={T}')
+
+    def heads(*shape):
+        return torch.randn(*shape, T, 8, 64, device=DEV, generator=g)
+    raw, a, fixed, values, target = heads(b), heads(n, b).bfloat16(), heads(b).bfloat16(), heads(b).bfloat16(), heads(b)
+    cos, sin = torch.randn(T, 32, device=DEV, generator=g), torch.randn(T, 32, device=DEV, generator=g)
+    args = (kind, raw, a, 0.5, cos, sin, fixed, values, window)
+    out = credit.rerun(*args)
+    base = heads(b)
+    for base in (base, base.bfloat16(), base.transpose(1, 2).contiguous().transpose(1, 2),
+                 torch.cat([base.new_zeros(1), base.flatten()])[1:].view(base.shape)):
+        ref = credit.head_scores(out, base, target)
+        got = credit.rerun_scores(*args, base, target)
+        change = (out.double() - base.double()) * target.double()
+        bound = 64 * 2 ** -23 * change.abs().sum(-1).permute(1, 3, 2, 0) + 1e-30
+        assert got.shape == ref.shape and ((got.double() - ref.double()).abs() <= bound).all()
