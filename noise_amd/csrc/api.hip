@@ -125,7 +125,7 @@ int noise_lowrank_linear(const void* x, long x_ld, long x_mstride, const void* w
   Carve c(workspace);
   float* u = c.take<float>((size_t)members * T);
   const int M = members * T;
-  if (int rc = rowdot_launch(static_cast<const bf16*>(x), x_ld, x_mstride, M, in, T, pair_shift, b, in, u, s))
+  if (int rc = rowdot_launch(RowdotArgs{static_cast<const bf16*>(x), x_ld, x_mstride, M, in, T, pair_shift, b, in, u}, s))
     return rc;
   LowrankGemmArgs g = base_args(x, x_ld, x_mstride, w, in, out, a, sign, members, T, pair_shift);
   g.u = u;
@@ -166,8 +166,9 @@ int noise_lowrank_mlp(const void* x, long x_ld, long x_mstride, const void* w_fc
   float* upart = c.take<float>(M * parts);
   bf16* hid = c.take<bf16>(M * f);
   bf16* wpt = c.take<bf16>((size_t)d * f);
-  if (int rc = rowdot_launch(static_cast<const bf16*>(x), x_ld, x_mstride, (int)M, d, T, pair_shift, b_fc, d, u_fc, s))
-    return rc;
+  // the input-side dots of c_fc, and w_proj's copy into WTILE for c_proj, in one launch
+  const RowdotArgs dots{static_cast<const bf16*>(x), x_ld, x_mstride, (int)M, d, T, pair_shift, b_fc, d, u_fc};
+  if (int rc = rowdot_tiles_launch(dots, static_cast<const bf16*>(w_proj), d, f, wpt, s)) return rc;
   LowrankGemmArgs g1 = base_args(x, x_ld, x_mstride, w_fc, d, f, a_fc, sign, members, T, pair_shift);
   g1.u = u_fc;
   g1.u_parts = 1;
@@ -181,7 +182,6 @@ int noise_lowrank_mlp(const void* x, long x_ld, long x_mstride, const void* w_fc
   g1.upart_ld = parts;
   if (int rc = lowrank_gemm_launch(EPI_RELU2, g1, s)) return rc;
   // c_proj loads both operands as whole 128-byte lines: the hidden in TILE16, w_proj copied into WTILE
-  if (int rc = weight_tiles_launch(static_cast<const bf16*>(w_proj), f, d, f, wpt, s)) return rc;
   LowrankGemmArgs g2 = base_args(hid, f, (long)T * f, wpt, f, d, a_proj, sign, members, T, pair_shift);
   g2.a_tiled = 1;
   g2.w_tiled = 1;

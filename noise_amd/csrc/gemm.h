@@ -112,6 +112,19 @@ struct LowrankGemmArgs {
   const float* col_scale;
 };
 
+// Row dots u[row] = bf16(sum_k x[row, k] bf16(b[dir, k])) of a bf16 activation, K % 8 == 0: the input-side half of `lowrank`.
+struct RowdotArgs {
+  const __bf16* x;
+  long ldx, x_mstride;  // row t of member p at x + p * x_mstride + t * ldx (x_mstride 0: one activation for all members)
+  int M, K, T, pair_shift;
+  const float* b;
+  long ldb;
+  float* u;
+};
+int rowdot_launch(const RowdotArgs& g, hipStream_t stream);
+// The same, and weight_tiles_launch (row-major w [N, K2] with row stride K2), in one launch.
+int rowdot_tiles_launch(const RowdotArgs& g, const __bf16* w, int N, int K2, __bf16* out, hipStream_t stream);
+
 // WTILE copy (out, N * K bf16) of a row-major bf16 weight in [N, K] with row stride ld.
 int weight_tiles_launch(const __bf16* in, long ld, int N, int K, __bf16* out, hipStream_t stream);
 // The fp16 operand of EPI_CE_F16 from an fp32 weight w [N, 512] (row stride ldw) and an optional gain [512]

@@ -646,11 +646,10 @@ int launch_epi(const LowrankGemmArgs& g, hipStream_t stream) {
 }  // namespace
 
 namespace {
-// WTILE copy of a row-major bf16 weight: thread q writes the 16-byte output chunk q (block q / 64, row r and
-// physical chunk p of the block), read from the weight row and logical chunk the layout assigns to it.
-__global__ void __launch_bounds__(256) weight_tiles_kernel(const bf16* __restrict__ in, long ld, int K, long chunks,
-                                                           bf16* __restrict__ out) {
-  const long q = (long)blockIdx.x * 256 + threadIdx.x;
+// WTILE copy of a row-major bf16 weight: the 16-byte output chunk q (block q / 64, row r and physical chunk p of the
+// block), read from the weight row and logical chunk the layout assigns to it.
+__device__ __forceinline__ void weight_tile_chunk(const bf16* __restrict__ in, long ld, int K, long chunks,
+                                                  bf16* __restrict__ out, long q) {
   if (q >= chunks) return;
   const long blk = q >> 6, kt = K >> 5, g = blk / kt, st = blk - g * kt;
   const int u = (int)(q & 63), r = u >> 2, c = (u & 3) ^ ((r >> 1) & 3);
@@ -658,12 +657,111 @@ __global__ void __launch_bounds__(256) weight_tiles_kernel(const bf16* __restric
   const long n = (i & ~63L) + (r >> 2) * 16 + ((i & 63) >> 4) * 4 + (r & 3);
   *reinterpret_cast<uint4*>(out + 8 * q) = *reinterpret_cast<const uint4*>(in + n * ld + 32 * st + 8 * c);
 }
+__global__ void __launch_bounds__(256) weight_tiles_kernel(const bf16* __restrict__ in, long ld, int K, long chunks,
+                                                           bf16* __restrict__ out) {
+  weight_tile_chunk(in, ld, K, chunks, out, (long)blockIdx.x * 256 + threadIdx.x);
+}
+
+// Rank-1 GEMV u[row] = bf16(x . bf16(b_dir)). A wave takes four rows of one member against its direction or, where every
+// member reads the same x, four rows against four directions (an antithetic pair's two members share the dot): each b
+// is read once per four rows and each x row once per four directions instead of both for every dot. Bound by the traffic
+// out of L2: 256 members (128 pairs) x 2048 tokens on one x 81.5 us with a wave per row, 27.1 now
+// with the weight copy (5.5) in the same launch. A lane adds its 8
+// columns in order and the lanes' sums meet in one tree, whatever the grouping.
+template <int DB>
+__device__ __forceinline__ void rowdot_units(const RowdotArgs& g, int wave, int nwaves) {
+  constexpr int RB = 4;
+  const int lane = threadIdx.x & 63;
+  const int members = g.M / g.T, dirs = (members + (1 << g.pair_shift) - 1) >> g.pair_shift;
+  const int rt = (g.T + RB - 1) / RB, units = rt * (DB == 1 ? members : (dirs + DB - 1) / DB);
+  for (int unit = wave; unit < units; unit += nwaves) {
+    const int first = unit / rt, t0 = (unit - first * rt) * RB;  // member, or group of DB directions
+    const int dir0 = DB == 1 ? first >> g.pair_shift : first * DB;
+    const bf16* xr[RB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+      xr[r] = g.x + (DB == 1 ? (long)first * g.x_mstride : 0) + (long)min(t0 + r, g.T - 1) * g.ldx;
+    float acc[RB][DB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r)
+#pragma unroll
+      for (int d = 0; d < DB; ++d) acc[r][d] = 0.f;
+    for (int k = lane * 8; k < g.K; k += 512) {
+      bf16x8 xv[RB];
+#pragma unroll
+      for (int r = 0; r < RB; ++r) xv[r] = *reinterpret_cast<const bf16x8*>(xr[r] + k);
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+        const float* br = g.b + (long)min(dir0 + d, dirs - 1) * g.ldb + k;
+        const float4 b0 = *reinterpret_cast<const float4*>(br), b1 = *reinterpret_cast<const float4*>(br + 4);
+        const float bv[8] = {bf16r(b0.x), bf16r(b0.y), bf16r(b0.z), bf16r(b0.w),
+                             bf16r(b1.x), bf16r(b1.y), bf16r(b1.z), bf16r(b1.w)};
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+          float t = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) t += (float)xv[r][e] * bv[e];
+          acc[r][d] += t;
+        }
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < DB; ++d)
+#pragma unroll
+      for (int r = 0; r < RB; ++r) {
+        const float u = bf16r(group_sum<64>(acc[r][d]));
+        if (lane || t0 + r >= g.T || dir0 + d >= dirs) continue;
+        if (DB == 1) {
+          g.u[(long)first * g.T + t0 + r] = u;
+        } else {
+          for (int p = (dir0 + d) << g.pair_shift; p < min(members, (dir0 + d + 1) << g.pair_shift); ++p)
+            g.u[(long)p * g.T + t0 + r] = u;
+        }
+      }
+  }
+}
+// Workgroups 0 .. tile_blocks - 1 copy w into WTILE, the others take the row dots.
+template <int DB>
+__global__ void __launch_bounds__(256) rowdot_kernel(RowdotArgs g, int tile_blocks, const bf16* __restrict__ w, int K2,
+                                                     long chunks, bf16* __restrict__ out) {
+  const int b = blockIdx.x - tile_blocks;
+  if (b < 0)
+    weight_tile_chunk(w, K2, K2, chunks, out, (long)blockIdx.x * 256 + threadIdx.x);
+  else
+    rowdot_units<DB>(g, b * 4 + (threadIdx.x >> 6), (gridDim.x - tile_blocks) * 4);
+}
+int rowdot_any(const RowdotArgs& g, int tile_blocks, const bf16* w, int K2, long chunks, bf16* out, hipStream_t stream) {
+  if (!g.x || !g.b || !g.u || g.M <= 0 || g.K <= 0 || g.K % 8 || g.ldx % 8 || g.x_mstride % 8 || g.ldb % 4 || g.T <= 0 ||
+      g.M % g.T)
+    return NOISE_EINVAL;
+  const int members = g.M / g.T, dirs = (members + (1 << g.pair_shift) - 1) >> g.pair_shift, rt = (g.T + 3) / 4;
+  const bool shared = g.x_mstride == 0 && members > 1;
+  const long units = (long)rt * (shared ? (dirs + 3) / 4 : members);
+  const unsigned grid = (unsigned)(tile_blocks + std::min<long>((units + 3) / 4, 8192));
+  if (shared)
+    hipLaunchKernelGGL(rowdot_kernel<4>, dim3(grid), dim3(256), 0, stream, g, tile_blocks, w, K2, chunks, out);
+  else
+    hipLaunchKernelGGL(rowdot_kernel<1>, dim3(grid), dim3(256), 0, stream, g, tile_blocks, w, K2, chunks, out);
+  NOISE_CHECK_LAUNCH();
+  return NOISE_OK;
+}
+bool bad_tiles(const bf16* in, long ld, int N, int K, const bf16* out) {
+  return !in || !out || N <= 0 || K <= 0 || N % 64 || K % 32 || ld < K || ld % 8 ||
+         (((uintptr_t)in | (uintptr_t)out) & 15);
+}
 }  // namespace
 
+int rowdot_launch(const RowdotArgs& g, hipStream_t stream) { return rowdot_any(g, 0, nullptr, 0, 0, nullptr, stream); }
+
+int rowdot_tiles_launch(const RowdotArgs& g, const bf16* w, int N, int K2, bf16* out, hipStream_t stream) {
+  if (bad_tiles(w, K2, N, K2, out)) return NOISE_EINVAL;
+  const long chunks = (long)N * K2 / 8, blocks = (chunks + 255) / 256;
+  if (blocks > 0x7fff0000L) return NOISE_ENOTSUP;
+  return rowdot_any(g, (int)blocks, w, K2, chunks, out, stream);
+}
+
 int weight_tiles_launch(const bf16* in, long ld, int N, int K, bf16* out, hipStream_t stream) {
-  if (!in || !out || N <= 0 || K <= 0 || N % 64 || K % 32 || ld < K || ld % 8 ||
-      (((uintptr_t)in | (uintptr_t)out) & 15))
-    return NOISE_EINVAL;
+  if (bad_tiles(in, ld, N, K, out)) return NOISE_EINVAL;
   const long chunks = (long)N * K / 8;
   hipLaunchKernelGGL(weight_tiles_kernel, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, stream, in, ld, K,
                      chunks, out);

@@ -134,6 +134,3 @@ struct CastBatchArgs {
   int n;
 };
 int cast_batch_launch(const CastMat* mats, int n, hipStream_t s);
-// Row dots u[row] = bf16(sum_k x[row, k] * bf16(b[dir, k])) for a bf16 activation.
-int rowdot_launch(const __bf16* x, long ldx, long x_mstride, int M, int K, int T, int pair_shift,
-                  const float* b, long ldb, float* u, hipStream_t stream);

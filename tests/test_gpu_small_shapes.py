@@ -432,3 +432,30 @@ def test_scores_of_a_credit_chunk_equal_those_of_its_outputs(kind, n, b, T, wind
         change = (out.double() - base.double()) * target.double()
         bound = 64 * 2 ** -23 * change.abs().sum(-1).permute(1, 3, 2, 0) + 1e-30
         assert got.shape == ref.shape and ((got.double() - ref.double()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize('members,T,pair', [(1, 1, 0), (2, 7, 1), (5, 33, 1), (9, 130, 0), (18, 4, 1)])
+@pytest.mark.parametrize('din', [64, 512, 1088])
+def test_linear_on_shared_activations_equals_separate_copies(members, T, pair, din):
+    """The input-side dots take four rows against one direction, or against four where members share one activation:
+    the same bits, for ragged row and direction groups, odd member counts and pairs."""
+    from noise_amd import ops
+    g = torch.Generator(DEV).manual_seed(46)
+    log_case(f'linear on shared activations members={members} T={T} pair={pair} din={din}')
+    dirs = (members + pair) >> pair
+    x = torch.randn(T, din, device=DEV, generator=g).bfloat16()
+    w = (torch.randn(128, din, device=DEV, generator=g) * din ** -0.5).bfloat16()
+    a, b = torch.randn(dirs, 128, device=DEV, generator=g), torch.randn(dirs, din, device=DEV, generator=g)
+    sign = torch.randn(members, device=DEV, generator=g)
+    one = ops.lowrank_linear(x, w, a, b, sign, T=T, pair_shift=pair)
+    own = ops.lowrank_linear(x[None].repeat(members, 1, 1).contiguous(), w, a, b, sign, T=T, pair_shift=pair)
+    assert torch.equal(one, own)
+    xd, wd, s = x.double(), w.double(), sign.double()[:, None, None]
+    pick = torch.arange(members, device=DEV) >> pair
+    av, bv = a.double()[pick][:, None], b.bfloat16().double()[pick]
+    dense, u = xd @ wd.t(), (xd @ bv.t()).t()[..., None]
+    ref = dense + s * u * av
+    # the dense product and the dot are each rounded to bf16 (2^-8) after din fp32 additions
+    mag = xd.abs() @ wd.abs().t() + s.abs() * (xd.abs() @ bv.abs().t()).t()[..., None] * av.abs()
+    bound = 1.01 * 2 ** -8 * (dense.abs() + (s * u * av).abs()) + (din + 4) * 2 ** -23 * mag
+    assert ((one.double() - ref).abs() <= bound).all()
