@@ -641,7 +641,11 @@ int block_entry_launch(const BlockEntryArgs& g, hipStream_t s) {
   if (g.gate_w && (!g.gate_a || !g.gate_b || !g.gate || (((uintptr_t)g.gate_w | (uintptr_t)g.gate_b) & 15)))
     return NOISE_EINVAL;
   if (bad_pending(g.pend, g.npend)) return NOISE_EINVAL;
-  const bool first = !g.x_in && !g.x0 && !g.npend, grouped = g.T % GROUP_ROWS == 0 && g.M % GROUP_ROWS == 0;
+  // a wave per row up to 32 rows per CU: a workgroup of 8 rows then holds its CU alone for two row latencies and the
+  // staging of its vectors (256 rows 7.8 -> 5.0 us, 2048 9.0 -> 6.5, 8192 15.2 -> 14.3; at 32,768 block 0 loses, 30.9 ->
+  // 34.4)
+  const bool first = !g.x_in && !g.x0 && !g.npend;
+  const bool grouped = g.T % GROUP_ROWS == 0 && g.M % GROUP_ROWS == 0 && g.M > 32 * num_cus();
   if (first && grouped)
     hipLaunchKernelGGL(block_entry_group_kernel<true>, dim3((unsigned)(g.M / GROUP_ROWS)), dim3(256), 0, s, g);
   else if (first)

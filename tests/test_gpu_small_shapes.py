@@ -459,3 +459,40 @@ def test_linear_on_shared_activations_equals_separate_copies(members, T, pair, d
     mag = xd.abs() @ wd.abs().t() + s.abs() * (xd.abs() @ bv.abs().t()).t()[..., None] * av.abs()
     bound = 1.01 * 2 ** -8 * (dense.abs() + (s * u * av).abs()) + (din + 4) * 2 ** -23 * mag
     assert ((one.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize('first', [False, True])
+@pytest.mark.parametrize('T', [136, 1096])
+def test_block_entry_of_few_and_many_rows_agree_bit_for_bit(T, first):
+    """Past 32 rows per CU the block entry runs workgroups of 8 rows, below it a wave per row: every member's stream,
+    operand, dots and gates are the same bits in a launch of more than 16,000 rows and in one of its own."""
+    g = torch.Generator(DEV).manual_seed(48)
+    m, D, V = 16384 // T + 2, 512, 640
+    M = m * T
+    log_case(f'block entry of few and many rows T={T} first={first}')
+
+    def rnd(*shape):
+        return torch.randn(*shape, device=DEV, generator=g)
+    x, y1, y2, u1, u2 = rnd(M, D), rnd(M, D).bfloat16(), rnd(M, D).bfloat16(), rnd(M, 8), rnd(M, 8)
+    v = {k: rnd(m, n) for k, n in dict(a1=D, a2=D, er=1, e0=1, bq=D, bk=D, bv=D, ga=8, gb=32, ea=V, eb=D).items()}
+    gw, w, lr, l0, sign = rnd(8, 32), rnd(V, D), rnd(1), rnd(1), 0.1 * rnd(m)
+    idx = torch.randint(0, V, (T,), device=DEV, generator=g)
+
+    def run(lo, hi):
+        n, r = (hi - lo) * T, slice(lo * T, hi * T)
+        xo, h = torch.empty(n, D, device=DEV), torch.empty(n, D, device=DEV, dtype=torch.bfloat16)
+        u, gate = torch.empty(n, 4, device=DEV), torch.empty(n, 8, device=DEV)
+        d = {k: t[lo:].data_ptr() for k, t in v.items()}
+        pend, npend = _lib.pending((y1[r].data_ptr(), u1[r].data_ptr(), 8, 8, 1, d['a1']),
+                                   (y2[r].data_ptr(), u2[r].data_ptr(), 8, 8, 1, d['a2']))
+        _emb, emb = _lib.embed(w.data_ptr(), V, d['ea'], d['eb'], idx.data_ptr(), 0)
+        _lib.call('noise_block_entry', None if first else x[r].data_ptr(), None, xo.data_ptr(), h.data_ptr(),
+                  u.data_ptr(), d['bq'], d['bk'], d['bv'], lr.data_ptr(), l0.data_ptr(), d['er'], d['e0'], 1,
+                  gw.data_ptr(), d['ga'], d['gb'], gate.data_ptr(), sign[lo:].data_ptr(), hi - lo, T, 0,
+                  None if first else pend, 0 if first else npend, emb, _stream())
+        torch.cuda.synchronize()
+        return xo, h, u, gate
+    whole = run(0, m)
+    for lo in (0, m // 2, m - 1):
+        for one, all_ in zip(run(lo, lo + 1), whole):
+            assert torch.equal(one, all_[lo * T:(lo + 1) * T])
