@@ -496,3 +496,22 @@ def test_block_entry_of_few_and_many_rows_agree_bit_for_bit(T, first):
     for lo in (0, m // 2, m - 1):
         for one, all_ in zip(run(lo, lo + 1), whole):
             assert torch.equal(one, all_[lo * T:(lo + 1) * T])
+
+
+@pytest.mark.parametrize('T', [128, 1152, 2048])
+def test_moment_partials_around_eight(T):
+    """1, 9 and 16 partials per head: the moments are the fixed-order fp32 sums of y and y^2 per 128 queries, within fp32
+    rounding of fp64 means of the kernel's own output."""
+    g = torch.Generator(DEV).manual_seed(47)
+    log_case(f'moments T={T}')
+    x = torch.randn(T, 3, 512, device=DEV, generator=g).bfloat16()
+    x[:, 2] = x[:, 2].half().view(torch.bfloat16)
+    y, mom = torch.empty(T, 512, device=DEV, dtype=torch.bfloat16), torch.empty(1, 8, 2, 64, device=DEV)
+    n = _lib.size_query('noise_attention_workspace_size', 1, T)
+    ws = torch.empty(n, device=DEV, dtype=torch.uint8)
+    _lib.call('noise_attention', x.data_ptr(), 1, T, T, 0, _lib.QK_BF16, None, 0, y.data_ptr(), None, mom.data_ptr(),
+              ws.data_ptr(), n, _stream())
+    torch.cuda.synchronize()
+    yd = y.double().view(T, 8, 64)
+    ref, mag = torch.stack([yd.mean(0), yd.square().mean(0)], 1), torch.stack([yd.abs().mean(0), yd.square().mean(0)], 1)
+    assert ((mom[0].double() - ref).abs() <= (T // 128 + 12) * 2 ** -23 * mag).all()
