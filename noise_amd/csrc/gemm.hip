@@ -153,7 +153,7 @@ lowrank_gemm_kernel(const LowrankGemmArgs g) {
     for (int d = 0; d < C::LA; ++d) {
       if (g.a_tiled) {
         // the 16 rows of this instruction are one 1 KiB TILE16 tile per 32-deep stage
-        const int G = min(m0 + (wave * C::LA + d) * C::ROWS_PER_DMA, g.M - 16) >> 4;
+        const int G = min((m0 >> 4) + wave * C::LA + d, (g.M - 1) >> 4);
         a_src[d] = (long)G * 16 * g.lda + 8 * lane;
       } else {
         const int r = (wave * C::LA + d) * C::ROWS_PER_DMA + lrow;
@@ -834,7 +834,9 @@ int lowrank_gemm_parts(int N) {
 }
 
 int lowrank_gemm_launch(int epi, const LowrankGemmArgs& g, hipStream_t stream) {
-  if (g.a_tiled && (epi == EPI_RELU2 || g.M % 16 || g.T % 16 || g.lda % 32 || g.a_mstride != (long)g.T * g.lda))
+  // (the fp16 head's own operand may end in a partial 16-row group, stored whole; a caller's may not)
+  if (g.a_tiled && (epi == EPI_RELU2 || g.lda % 32 || g.a_mstride != (long)g.T * g.lda ||
+                    (epi != EPI_CE_F16 && (g.M % 16 || g.T % 16))))
     return NOISE_EINVAL;
   if (g.out_tiled && (epi != EPI_RELU2 || g.M % 16 || g.ldo % 32)) return NOISE_EINVAL;
   if (epi == EPI_DENSE) {

@@ -382,12 +382,13 @@ __global__ void __launch_bounds__(1024) head_norm_tiled_kernel(HeadNormArgs g) {
   const int lane = threadIdx.x & 63, r16 = threadIdx.x >> 6;
   const long r0 = (long)blockIdx.x * 16, row = r0 + r16;
   const int W = g.fp32_head == 1 ? 2 * D : D, units = W / 8;
-  const int p = (int)(row / g.T), dir = p >> g.pair_shift;
+  const long live = min(row, (long)g.M - 1);  // (rows past the last fill its group with copies, which nothing reads)
+  const int p = (int)(live / g.T), dir = p >> g.pair_shift;
   u32x4 op[2];
-  const float u = head_operand(g, head_row(g, row, lane, p, dir), lane, dir, op);
+  const float u = head_operand(g, head_row(g, live, lane, p, dir), lane, dir, op);
   rows16[r16][lane] = op[0];
   if (g.fp32_head == 1) rows16[r16][64 + lane] = op[1];
-  if (lane == 0) g.u[row] = u;
+  if (lane == 0 && row < g.M) g.u[row] = u;
   __syncthreads();
   // unit n of the group: tile n / 64, q = n % 64 -> row q / 4, 8-column chunk (q % 4) ^ ((q / 8) % 4) of the tile
   bf16* out = g.h + r0 * W;
@@ -671,8 +672,7 @@ int head_norm_launch(const HeadNormArgs& g, hipStream_t s) {
       (g.x_bf16 && g.npend) || g.fp32_head < 0 || g.fp32_head > 2)
     return NOISE_EINVAL;
   if (g.tiled) {
-    if (g.M % 16) return NOISE_EINVAL;
-    hipLaunchKernelGGL(head_norm_tiled_kernel, dim3((unsigned)(g.M / 16)), dim3(1024), 0, s, g);
+    hipLaunchKernelGGL(head_norm_tiled_kernel, dim3((unsigned)((g.M + 15L) / 16)), dim3(1024), 0, s, g);
   } else {
     hipLaunchKernelGGL(head_norm_kernel, dim3(grid_rows(g.M)), dim3(256), 0, s, g);
   }

@@ -515,3 +515,33 @@ def test_moment_partials_around_eight(T):
     yd = y.double().view(T, 8, 64)
     ref, mag = torch.stack([yd.mean(0), yd.square().mean(0)], 1), torch.stack([yd.abs().mean(0), yd.square().mean(0)], 1)
     assert ((mom[0].double() - ref).abs() <= (T // 128 + 12) * 2 ** -23 * mag).all()
+
+
+@pytest.mark.parametrize('members,T', [(1, 1), (3, 5), (2, 1501), (9, 333), (1, 2049)])
+def test_head_of_ragged_rows_from_tiled_and_row_major_operands(members, T):
+    """From 2048 rows on the fp32 head pads its tiled operand to whole 16-row groups; with a workspace that has no room for
+    the padding it takes row-major operands. The losses are the same bits, and a workspace smaller still is refused."""
+    g = torch.Generator(DEV).manual_seed(49)
+    V, M = 512, members * T
+    log_case(f'ragged fp32 head members={members} T={T}')
+    x, w = torch.randn(M, 512, device=DEV, generator=g), torch.randn(V, 512, device=DEV, generator=g) * 0.05
+    a, b = torch.randn(members, V, device=DEV, generator=g), torch.randn(members, 512, device=DEV, generator=g)
+    sign = 0.01 * torch.randn(members, device=DEV, generator=g)
+    tgt = torch.randint(0, V, (T,), device=DEV, generator=g)
+    full = _lib.size_query('noise_head_ce_workspace_size', members, T, V, _lib.HEAD_FP32)
+    least = full - (-M) % 16 * 1024
+    assert least < full
+    ws = torch.empty(full, device=DEV, dtype=torch.uint8)
+
+    def run(size):
+        loss = torch.full((M + 16,), 7., device=DEV)
+        _lib.call('noise_head_ce', x.data_ptr(), 0, None, w.data_ptr(), V, _lib.HEAD_FP32, a.data_ptr(), b.data_ptr(),
+                  sign.data_ptr(), tgt.data_ptr(), 0, members, T, 0, _lib.CE_NONE, loss.data_ptr(), None, ws.data_ptr(),
+                  size, None, 0, _stream())
+        torch.cuda.synchronize()
+        assert (loss[M:] == 7).all()
+        return loss[:M]
+    tiled = run(full)
+    assert torch.equal(tiled, run(least)) and torch.isfinite(tiled).all()
+    with pytest.raises(_lib.NoiseHipError, match='NOISE_ENOSPC'):
+        run(least - 1)
