@@ -88,10 +88,10 @@ __global__ void __launch_bounds__(256) fold_fitness_kernel(const float* __restri
 }
 
 // G[o, i] = scale * sum_j (w_j a_j[o]) b_j[i] over ndir directions (a null: a_j[o] = 1, out = 1), for up
-// to OUTER_MAX matrices in one launch, where they make fewer 128 x 128 tiles than CUs (outer_split_kernel otherwise). On the fp32 MFMA (v_mfma_f32_16x16x4_f32): a
-// 64 x 64 output tile per workgroup of 4 waves (32 x 32 each); directions pass through a double-buffered
-// LDS stage 32 at a time with w_j folded into the a rows, the next 32 loaded into registers while the
-// current ones feed the MFMAs.
+// to OUTER_MAX matrices in one launch, where they make fewer 128 x 128 tiles than CUs (outer_split_kernel otherwise). On
+// the fp32 MFMA (v_mfma_f32_16x16x4_f32): a 64 x 64 output tile per workgroup of 4 waves (32 x 32 each); directions pass
+// through a double-buffered LDS stage 32 at a time with w_j folded into the a rows, the next 32 loaded into registers
+// while the current ones feed the MFMAs.
 __global__ void __launch_bounds__(256) outer_update_kernel(const OuterBatchArgs g) {
   constexpr int TK = 32, LD = 64 + 4;
   __shared__ __attribute__((aligned(16))) float sa[2][TK][LD];
@@ -227,7 +227,9 @@ __global__ void __launch_bounds__(256, 2) outer_split_kernel(const OuterBatchArg
   const int o0 = (lt / M.tiles_i) * OS_TILE, i0 = (lt % M.tiles_i) * OS_TILE;
   // loader: directions 4 jg .. 4 jg + 3 of the 32, columns 4 q .. 4 q + 3 of the 128
   const int q = tid & 31, jg = tid >> 5;
-  const bool full = M.a && o0 + OS_TILE <= M.out && i0 + OS_TILE <= M.in;
+  // 16-byte loads only where every row starts at a 16-byte address
+  const bool full = M.a && o0 + OS_TILE <= M.out && i0 + OS_TILE <= M.in && M.a_ld % 4 == 0 && M.b_ld % 4 == 0 &&
+                    !(((uintptr_t)M.a | (uintptr_t)M.b) & 15);
   // the w factors stay apart until the rows are staged: a use here would wait for the loads
   float4 ra[4], rb[4];
   float rw[4];

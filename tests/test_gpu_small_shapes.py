@@ -336,6 +336,31 @@ def test_outer_update_on_split_operands(n):
         assert ((got.double() - ref).abs() <= bound).all()
 
 
+@pytest.mark.parametrize('pad,off', [(0, 1), (2, 0), (4, 3)])
+def test_outer_update_of_rows_off_16_byte_addresses(pad, off):
+    """Full 128 x 128 tiles whose rows start off 16-byte addresses (by the pointer, the row stride or both): the bits of
+    the aligned rows."""
+    g = torch.Generator().manual_seed(43)
+    log_case(f'outer update, row padding {pad}, offset {off}')
+    n, o, i = 37, 4096, 1024
+    a, b, w = (torch.randn(n, k, generator=g).to(DEV) for k in (o, i, 1))
+    got = []
+    for p, f in ((0, 0), (pad, off)):
+        rows = []
+        for t in (a, b):
+            flat = torch.zeros(n * (t.shape[1] + p) + f, device=DEV)
+            rows.append(flat[f:].view(n, -1)[:, :t.shape[1]])
+            rows[-1].copy_(t)
+        grad = torch.zeros(o, i, device=DEV)
+        ptr, cnt, _keep = _lib.outer_mats([(rows[0].data_ptr(), o + p, rows[1].data_ptr(), i + p, o, i, grad.data_ptr())])
+        _lib.call('noise_outer_update_batch', ptr, cnt, w.data_ptr(), n, 1.0, _stream())
+        got.append(grad)
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], got[1])
+    ref = (a * w).double().cpu().t() @ b.double().cpu()
+    assert (got[0].cpu().double() - ref).norm() <= 1e-6 * ref.norm()
+
+
 def test_outer_update_of_non_finite_and_extreme_values():
     """Infinities, NaN and values that bf16 would round to infinity: what the fp32 sum gives, in that column or row only;
     tiny values (a product of 1e-30) keep their sum."""
