@@ -616,8 +616,8 @@ bool use_big(int N) { return N % 256 == 0; }
 //  - 64 x 64 tiles while at most three of them fall on a CU: a larger tile then leaves most CUs idle behind one long K
 //    chain (2048 x 512 outputs, K = 2048: 42.9 us on 16 tiles of 256 x 256, 20.9 on 64 of 128 x 128, 10.7 on 256 of
 //    64 x 64; 6144 rows, three per CU: 43.4, 22.2, 20.4; 8192 rows, four per CU: 43.7, 23.3, 25.9). Its steps are bound by
-//    their own chain (barrier, LDS reads, MFMAs: 164 ns each), not by loads in flight: rings of 6 and 8 stages instead of
-//    4 took 11.5 and 11.2 us against 10.5 in those 256 tiles.
+//    their own chain (LDS reads, MFMAs: 164 ns each), not by loads in flight or barriers: rings of 6 and 8 stages instead
+//    of 4 took 11.5 and 11.2 us against 10.5 in those 256 tiles, 8 stages opened two at a time 10.9.
 //  - beyond that, the fewer rounds of the GPU. In units of one round of 256 x 256 tiles (one workgroup per CU, 55.7 us
 //    at K = 2048), 128 x 128 tiles, two workgroups per CU, cost 0.585 a full round and 0.36 where the last one leaves
 //    one per CU; 256 x 128 tiles (N not a multiple of 256) 0.56. So 128 x 128 tiles run ragged ends (16384 rows: 47.4
