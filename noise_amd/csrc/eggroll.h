@@ -16,8 +16,8 @@ struct OuterUpdateArgs {
 };
 
 // Kernel-side form: up to OUTER_MAX matrices per launch, passed by value (under the 4 KiB argument limit),
-// with the running total of 64 x 64 tiles.
-constexpr int OUTER_MAX = 64;
+// with the running total of OUTER_TILE x OUTER_TILE tiles.
+constexpr int OUTER_MAX = 64, OUTER_TILE = 64;
 struct OuterMat {
   const float* a;
   const float* b;

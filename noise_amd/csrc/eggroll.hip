@@ -88,132 +88,25 @@ __global__ void __launch_bounds__(256) fold_fitness_kernel(const float* __restri
 }
 
 // G[o, i] = scale * sum_j (w_j a_j[o]) b_j[i] over ndir directions (a null: a_j[o] = 1, out = 1), for up
-// to OUTER_MAX matrices in one launch, where they make fewer 128 x 128 tiles than CUs (outer_split_kernel otherwise). On
-// the fp32 MFMA (v_mfma_f32_16x16x4_f32): a 64 x 64 output tile per workgroup of 4 waves (32 x 32 each); directions pass
-// through a double-buffered LDS stage 32 at a time with w_j folded into the a rows, the next 32 loaded into registers
-// while the current ones feed the MFMAs.
-__global__ void __launch_bounds__(256) outer_update_kernel(const OuterBatchArgs g) {
-  constexpr int TK = 32, LD = 64 + 4;
+// to OUTER_MAX matrices in one launch (every perturbed parameter of the model: ~9k 64 x 64 tiles fill the
+// GPU, where one 512 x 512 matrix alone is 64 workgroups). On the fp32 MFMA (v_mfma_f32_16x16x4_f32): a
+// 64 x 64 output tile per workgroup of 4 waves (32 x 32 each); directions pass through a double-buffered
+// LDS stage 32 at a time with w_j folded into the a rows, the next 32 loaded into registers while the
+// current ones feed the MFMAs. Every output adds its directions four at a time in increasing order, so a matrix's
+// gradient is the same bits alone and beside any others, and infinities and NaN go where the fp32 sum takes them.
+// Bound by the fp32 MFMA: the model's 37.7M weights and 1536 directions (116 GFLOP) take 1100 us, 105 TFLOP/s of 157.
+// Before, one branch per operand row made each load wait for the last, and the w factors waited for the a rows: 1275 us.
+// (128 x 128 tiles, half the operand traffic, measured the same, 1083, and lose where tiles are few or ragged. Three bf16
+// planes per operand on the bf16 MFMA take 677, with a smaller error at these sizes, but hold fewer bits of operands
+// below 2^-110 and give bits that depend on whether the launch fills the GPU.)
+// LDS rows of 64 + 16 floats: the four directions of an MFMA operand fall in four different quarters of the banks.
+__global__ void __launch_bounds__(256, 2) outer_update_kernel(const OuterBatchArgs g) {
+  constexpr int TILE = OUTER_TILE, TK = 32, LD = TILE + 16, W = TILE / 2, F = W / 16, Q = TILE / 32;
   __shared__ __attribute__((aligned(16))) float sa[2][TK][LD];
   __shared__ __attribute__((aligned(16))) float sb[2][TK][LD];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  // this workgroup's matrix and tile (uniform scan over the prefix sums of tile counts)
-  const int t = blockIdx.x;
-  int mi = 0;
-  while (mi + 1 < g.n && t >= g.m[mi].tile_end) ++mi;
-  const OuterMat& M = g.m[mi];
-  const int lt = t - (mi ? g.m[mi - 1].tile_end : 0);
-  const int o0 = (lt / M.tiles_i) * 64, i0 = (lt % M.tiles_i) * 64;
-  // loader: thread tid fills direction jj = tid / 8 (of 32), columns 8 (tid % 8) .. + 7 of a and of b
-  const int ljj = tid >> 3, lc = 8 * (tid & 7);
-  const bool a_full = M.a && o0 + 64 <= M.out && M.a_ld % 4 == 0, b_full = i0 + 64 <= M.in && M.b_ld % 4 == 0;
-  float ra[8], rb[8];
-  auto load = [&](int j0) {
-    const int j = j0 + ljj;
-    const bool live = j < g.ndir;
-    const float wj = live ? g.w[j] : 0.f;
-    if (live && a_full) {
-      const float4 x0 = *reinterpret_cast<const float4*>(M.a + (long)j * M.a_ld + o0 + lc);
-      const float4 x1 = *reinterpret_cast<const float4*>(M.a + (long)j * M.a_ld + o0 + lc + 4);
-      ra[0] = x0.x, ra[1] = x0.y, ra[2] = x0.z, ra[3] = x0.w, ra[4] = x1.x, ra[5] = x1.y, ra[6] = x1.z, ra[7] = x1.w;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        ra[e] = live && o0 + lc + e < M.out ? (M.a ? M.a[(long)j * M.a_ld + o0 + lc + e] : 1.f) : 0.f;
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ra[e] *= wj;
-    if (live && b_full) {
-      const float4 x0 = *reinterpret_cast<const float4*>(M.b + (long)j * M.b_ld + i0 + lc);
-      const float4 x1 = *reinterpret_cast<const float4*>(M.b + (long)j * M.b_ld + i0 + lc + 4);
-      rb[0] = x0.x, rb[1] = x0.y, rb[2] = x0.z, rb[3] = x0.w, rb[4] = x1.x, rb[5] = x1.y, rb[6] = x1.z, rb[7] = x1.w;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) rb[e] = live && i0 + lc + e < M.in ? M.b[(long)j * M.b_ld + i0 + lc + e] : 0.f;
-    }
-  };
-  auto stage = [&](int buf) {
-    *reinterpret_cast<float4*>(&sa[buf][ljj][lc]) = make_float4(ra[0], ra[1], ra[2], ra[3]);
-    *reinterpret_cast<float4*>(&sa[buf][ljj][lc + 4]) = make_float4(ra[4], ra[5], ra[6], ra[7]);
-    *reinterpret_cast<float4*>(&sb[buf][ljj][lc]) = make_float4(rb[0], rb[1], rb[2], rb[3]);
-    *reinterpret_cast<float4*>(&sb[buf][ljj][lc + 4]) = make_float4(rb[4], rb[5], rb[6], rb[7]);
-  };
-  f32x4 acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  load(0);
-  stage(0);
-  __syncthreads();
-  int buf = 0;
-  for (int j0 = 0; j0 < g.ndir; j0 += TK) {
-    const bool more = j0 + TK < g.ndir;
-    if (more) load(j0 + TK);  // in flight during this chunk's MFMAs
-#pragma unroll
-    for (int ks = 0; ks < TK / 4; ++ks) {
-      const int jj = 4 * ks + (lane >> 4);
-      float af[2], bf[2];
-#pragma unroll
-      for (int f = 0; f < 2; ++f) {
-        af[f] = sa[buf][jj][wm * 32 + 16 * f + (lane & 15)];
-        bf[f] = sb[buf][jj][wn * 32 + 16 * f + (lane & 15)];
-      }
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[a], bf[b], acc[a][b], 0, 0, 0);
-    }
-    if (more) {
-      // the other buffer was last read in the previous chunk, before the barrier that ended it
-      stage(buf ^ 1);
-      __syncthreads();
-      buf ^= 1;
-    }
-  }
-  // lane holds C[row = 4 (lane / 16) + e][col = lane % 16] of each 16 x 16 block
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int o = o0 + wm * 32 + 16 * a + 4 * (lane >> 4) + e, i = i0 + wn * 32 + 16 * b + (lane & 15);
-        if (o < M.out && i < M.in) M.grad[(long)o * M.in + i] = g.scale * acc[a][b][e];
-      }
-}
-
-// The same sums on the bf16 MFMA, for updates that fill the GPU with 128 x 128 tiles. An fp32 value is
-// the sum of three bf16 (8 significant bits each: a1 = bf16(a), a2 = bf16(a - a1), a3 = bf16(a - a1 - a2), both
-// differences exact), and a b is a1 b1 + (a1 b2 + a2 b1) + (a1 b3 + a2 b2 + a3 b1) up to terms below 2^-25 |a b|, each
-// product exact in the fp32 accumulation. Six bf16 MFMAs of 32 directions take 96 cycles where eight fp32 ones take 256,
-// and the sum rounds 6 times per 32 directions instead of 8: its error against 64 bits is the smaller one at every
-// population measured (relative, N(0, 1) rows: 16 directions 5.5e-8 against 8.5e-8 of the fp32 kernel, 256 2.4e-7 against
-// 2.9e-7, 1536 6.1e-7 against 7.1e-7). The model's 37.7M weights: 1536 directions 1227 -> 656 us, 256 230 -> 129, 64
-// 93 -> 57, 16 68 -> 48.
-// A workgroup of 4 waves owns a 128 x 128 tile (64 x 64 per wave; half the operand traffic per product of 64 x 64 tiles,
-// which held the fp32 kernel at half its peak); the tiles of an XCD are consecutive, so the tiles of a matrix share its
-// a and b in that L2. A thread loads 4 directions x 4 columns of each operand, 32 directions ahead, splits them in
-// registers and writes the planes transposed to rows of 32 directions. LDS row r of a plane sits in 64-byte slot (r % 4) ^
-// (r / 16 % 4) of its group of four, 16-byte chunk c at c ^ (r / 4 % 4): a fragment's 16 rows fall in distinct banks, and
-// a store's 64 lanes two to a bank.
-// Infinities and NaN (and values beyond bf16's largest, which round to infinity) do not survive the split as they would
-// an fp32 sum: a tile with a non-finite result is summed again in fp32.
-constexpr int OS_TILE = 128, OS_TK = 32, OS_PLANE = OS_TILE * OS_TK;
-__device__ __forceinline__ int os_row(int r) { return (r >> 2) * 128 + (((r & 3) ^ ((r >> 4) & 3)) << 5); }
-__device__ __forceinline__ int os_at(int r, int c) { return os_row(r) + ((c ^ ((r >> 2) & 3)) << 3); }
-__device__ __forceinline__ float bf16_hi(unsigned pair) { return __uint_as_float(pair & 0xffff0000u); }
-__device__ __forceinline__ float bf16_lo(unsigned pair) { return __uint_as_float(pair << 16); }
-__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
-  bf16x2 p = {to_bf16(a), to_bf16(b)};
-  return *reinterpret_cast<unsigned*>(&p);
-}
-__global__ void __launch_bounds__(256, 2) outer_split_kernel(const OuterBatchArgs g) {
-  __shared__ __attribute__((aligned(16))) bf16 sp[2][3][OS_PLANE];  // operand (0: b rows i, 1: w a rows o), plane
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, grp = lane >> 4;
   const int wi = wave & 1, wo = wave >> 1;
-  // XCD x takes a contiguous range of tiles
+  // XCD x takes a contiguous range of tiles: the tiles of a matrix share its a and b in that L2
   const unsigned G = gridDim.x, bl = blockIdx.x, x = bl & 7, qg = G >> 3, rg = G & 7;
   const int t = (int)(x * qg + min(x, rg) + (bl >> 3));
   int mi = 0, hi = g.n - 1;
@@ -224,121 +117,89 @@ __global__ void __launch_bounds__(256, 2) outer_split_kernel(const OuterBatchArg
   }
   const OuterMat& M = g.m[mi];
   const int lt = t - (mi ? g.m[mi - 1].tile_end : 0);
-  const int o0 = (lt / M.tiles_i) * OS_TILE, i0 = (lt % M.tiles_i) * OS_TILE;
-  // loader: directions 4 jg .. 4 jg + 3 of the 32, columns 4 q .. 4 q + 3 of the 128
-  const int q = tid & 31, jg = tid >> 5;
-  // 16-byte loads only where every row starts at a 16-byte address
-  const bool full = M.a && o0 + OS_TILE <= M.out && i0 + OS_TILE <= M.in && M.a_ld % 4 == 0 && M.b_ld % 4 == 0 &&
+  const int o0 = (lt / M.tiles_i) * TILE, i0 = (lt % M.tiles_i) * TILE;
+  // loader: thread tid fills direction jj = tid / 8 (of 32), columns 4 (tid % 8) + 32 q .. + 3 of a and of b; 16-byte
+  // loads only where every row starts at a 16-byte address
+  const int ljj = tid >> 3, lc = 4 * (tid & 7);
+  const bool full = M.a && o0 + TILE <= M.out && i0 + TILE <= M.in && M.a_ld % 4 == 0 && M.b_ld % 4 == 0 &&
                     !(((uintptr_t)M.a | (uintptr_t)M.b) & 15);
-  // the w factors stay apart until the rows are staged: a use here would wait for the loads
-  float4 ra[4], rb[4];
-  float rw[4];
-  auto load = [&](int j0) {
-    const int j = j0 + 4 * jg;
-    if (full && j0 + OS_TK <= g.ndir) {
+  float4 ra[Q], rb[Q];
+  float rw;  // apart from the a row until it is staged: a use here would wait for the loads
+  auto load_row = [&](float4 (&r)[Q], const float* row, int cols) {
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        rw[d] = g.w[j + d];
-        ra[d] = *reinterpret_cast<const float4*>(M.a + (long)(j + d) * M.a_ld + o0 + 4 * q);
-        rb[d] = *reinterpret_cast<const float4*>(M.b + (long)(j + d) * M.b_ld + i0 + 4 * q);
+    for (int q = 0; q < Q; ++q) {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = lc + 32 * q + e < cols ? (row ? row[lc + 32 * q + e] : 1.f) : 0.f;
+      r[q] = make_float4(v[0], v[1], v[2], v[3]);
+    }
+  };
+  auto load = [&](int j0) {
+    const int j = j0 + ljj;
+    const bool live = j < g.ndir;
+    const float *ap = M.a ? M.a + (long)j * M.a_ld + o0 : nullptr, *bp = M.b + (long)j * M.b_ld + i0;
+    rw = live ? g.w[j] : 0.f;
+    // one branch for both rows: with one each, the second row's loads waited for the first's
+    if (full && j0 + TK <= g.ndir) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        ra[q] = *reinterpret_cast<const float4*>(ap + lc + 32 * q);
+        rb[q] = *reinterpret_cast<const float4*>(bp + lc + 32 * q);
       }
       return;
     }
+    load_row(ra, ap, live ? M.out - o0 : 0);
+    load_row(rb, bp, live ? M.in - i0 : 0);
+  };
+  auto stage = [&](int buf) {
 #pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const bool live = j + d < g.ndir;
-      const int na = live ? M.out - o0 - 4 * q : 0, nb = live ? M.in - i0 - 4 * q : 0;
-      const float* ap = M.a ? M.a + (long)(j + d) * M.a_ld + o0 + 4 * q : nullptr;
-      const float* bp = M.b + (long)(j + d) * M.b_ld + i0 + 4 * q;
-      float av[4], bv[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        av[e] = e < na ? (ap ? ap[e] : 1.f) : 0.f;
-        bv[e] = e < nb ? bp[e] : 0.f;
-      }
-      rw[d] = live ? g.w[j + d] : 0.f;
-      ra[d] = make_float4(av[0], av[1], av[2], av[3]);
-      rb[d] = make_float4(bv[0], bv[1], bv[2], bv[3]);
+    for (int q = 0; q < Q; ++q) {
+      *reinterpret_cast<float4*>(&sa[buf][ljj][lc + 32 * q]) =
+          make_float4(ra[q].x * rw, ra[q].y * rw, ra[q].z * rw, ra[q].w * rw);
+      *reinterpret_cast<float4*>(&sb[buf][ljj][lc + 32 * q]) = rb[q];
     }
   };
-  // one column's four directions, split into the three planes: 8 bytes each
-  auto put = [&](int op, int row, float v0, float v1, float v2, float v3) {
-    bf16* p = &sp[op][0][os_at(row, jg >> 1) + 4 * (jg & 1)];
+  f32x4 acc[F][F];  // [i block][o block]: lane holds i = 4 grp + e, o = lane % 16 of each 16 x 16 block
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const unsigned lo = pack_bf16(v0, v1), hw = pack_bf16(v2, v3);
-      *reinterpret_cast<uint2*>(p + k * OS_PLANE) = make_uint2(lo, hw);
-      v0 -= bf16_lo(lo), v1 -= bf16_hi(lo), v2 -= bf16_lo(hw), v3 -= bf16_hi(hw);
-    }
-  };
-  auto stage = [&]() {
-    put(0, 4 * q, rb[0].x, rb[1].x, rb[2].x, rb[3].x);
-    put(0, 4 * q + 1, rb[0].y, rb[1].y, rb[2].y, rb[3].y);
-    put(0, 4 * q + 2, rb[0].z, rb[1].z, rb[2].z, rb[3].z);
-    put(0, 4 * q + 3, rb[0].w, rb[1].w, rb[2].w, rb[3].w);
-    put(1, 4 * q, ra[0].x * rw[0], ra[1].x * rw[1], ra[2].x * rw[2], ra[3].x * rw[3]);
-    put(1, 4 * q + 1, ra[0].y * rw[0], ra[1].y * rw[1], ra[2].y * rw[2], ra[3].y * rw[3]);
-    put(1, 4 * q + 2, ra[0].z * rw[0], ra[1].z * rw[1], ra[2].z * rw[2], ra[3].z * rw[3]);
-    put(1, 4 * q + 3, ra[0].w * rw[0], ra[1].w * rw[1], ra[2].w * rw[2], ra[3].w * rw[3]);
-  };
-  f32x4 acc[4][4];  // [i block][o block]: lane holds i = 4 grp + e, o = lane % 16 of each 16 x 16 block
+  for (int a = 0; a < F; ++a)
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < F; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
   load(0);
-  for (int j0 = 0; j0 < g.ndir; j0 += OS_TK) {
-    if (j0) __syncthreads();  // the previous planes have been read
-    stage();
-    __syncthreads();
-    if (j0 + OS_TK < g.ndir) load(j0 + OS_TK);  // in flight during this chunk's MFMAs
-    bf16x8 fb[4][3];
+  stage(0);
+  __syncthreads();
+  int buf = 0;
+  for (int j0 = 0; j0 < g.ndir; j0 += TK) {
+    const bool more = j0 + TK < g.ndir;
+    if (more) load(j0 + TK);  // in flight during this chunk's MFMAs
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int ks = 0; ks < TK / 4; ++ks) {
+      const int jj = 4 * ks + grp;
+      float bf[F], af[F];
 #pragma unroll
-      for (int k = 0; k < 3; ++k)
-        fb[a][k] = *reinterpret_cast<const bf16x8*>(&sp[0][k][os_at(64 * wi + 16 * a + (lane & 15), grp)]);
+      for (int f = 0; f < F; ++f) {
+        bf[f] = sb[buf][jj][wi * W + 16 * f + (lane & 15)];
+        af[f] = sa[buf][jj][wo * W + 16 * f + (lane & 15)];
+      }
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      bf16x8 fa[3];
+      for (int a = 0; a < F; ++a)
 #pragma unroll
-      for (int k = 0; k < 3; ++k)
-        fa[k] = *reinterpret_cast<const bf16x8*>(&sp[1][k][os_at(64 * wo + 16 * b + (lane & 15), grp)]);
-      // the smallest terms first
-#pragma unroll
-      for (int s = 2; s >= 0; --s)
-#pragma unroll
-        for (int k = 0; k <= s; ++k)
-#pragma unroll
-          for (int a = 0; a < 4; ++a) acc[a][b] = mfma16x16x32(fb[a][k], fa[s - k], acc[a][b]);
+        for (int b = 0; b < F; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[a], af[b], acc[a][b], 0, 0, 0);
+    }
+    if (more) {
+      // the other buffer was last read in the previous chunk, before the barrier that ended it
+      stage(buf ^ 1);
+      __syncthreads();
+      buf ^= 1;
     }
   }
-  bool bad = false;
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) bad |= !(fabsf(acc[a][b][e]) < INFINITY);
-  bad = __syncthreads_or(bad);
   const bool vec = M.in % 4 == 0 && !((uintptr_t)M.grad & 15);
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int a = 0; a < F; ++a)
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int o = o0 + 64 * wo + 16 * b + (lane & 15), i = i0 + 64 * wi + 16 * a + 4 * grp;
+    for (int b = 0; b < F; ++b) {
+      const int o = o0 + wo * W + 16 * b + (lane & 15), i = i0 + wi * W + 16 * a + 4 * grp;
       if (o >= M.out || i >= M.in) continue;
-      float v[4] = {acc[a][b][0], acc[a][b][1], acc[a][b][2], acc[a][b][3]};
-      if (bad) {
-        const int n = min(4, M.in - i);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float sum = 0.f;
-          for (int j = 0; j < g.ndir && e < n; ++j)
-            sum = fmaf(g.w[j] * (M.a ? M.a[(long)j * M.a_ld + o] : 1.f), M.b[(long)j * M.b_ld + i + e], sum);
-          v[e] = sum;
-        }
-      }
+      const f32x4 v = acc[a][b];
       float* out = M.grad + (long)o * M.in + i;
       if (vec) {
         *reinterpret_cast<float4*>(out) = make_float4(g.scale * v[0], g.scale * v[1], g.scale * v[2], g.scale * v[3]);
@@ -478,16 +339,7 @@ int outer_update_launch(const OuterUpdateArgs* mats, int n, const float* w, int 
     g.w = w;
     g.ndir = ndir;
     g.scale = scale;
-    auto tiles_of = [&](int tile) {
-      long tiles = 0;
-      for (int k = 0; k < g.n; ++k) {
-        OuterMat& m = g.m[k];
-        m.tiles_i = (m.in + tile - 1) / tile;
-        tiles += (long)((m.out + tile - 1) / tile) * m.tiles_i;
-        m.tile_end = (int)std::min(tiles, 0x7fffffffL);
-      }
-      return tiles;
-    };
+    long tiles = 0;
     for (int k = 0; k < g.n; ++k) {
       const OuterUpdateArgs& u = mats[base + k];
       if (!u.b || !u.grad || u.out <= 0 || u.in <= 0 || (!u.a && u.out != 1) || u.b_ld < u.in ||
@@ -495,17 +347,12 @@ int outer_update_launch(const OuterUpdateArgs* mats, int n, const float* w, int 
         return NOISE_EINVAL;
       OuterMat& m = g.m[k];
       m.a = u.a, m.b = u.b, m.grad = u.grad, m.a_ld = u.a_ld, m.b_ld = u.b_ld, m.out = u.out, m.in = u.in;
+      m.tiles_i = (u.in + OUTER_TILE - 1) / OUTER_TILE;
+      tiles += (long)((u.out + OUTER_TILE - 1) / OUTER_TILE) * m.tiles_i;
+      if (tiles > 0x7fffffffL) return NOISE_ENOTSUP;
+      m.tile_end = (int)tiles;
     }
-    long tiles = tiles_of(OS_TILE);
-    // at least one 128 x 128 tile per CU: below that the smaller tiles of the fp32 kernel fill the GPU better (one
-    // 512 x 512 matrix, 1536 directions: 67 us on 64 tiles against 89 on 16)
-    const bool split = tiles >= num_cus();
-    if (!split) tiles = tiles_of(64);
-    if (tiles > 0x7fffffffL) return NOISE_ENOTSUP;
-    if (split)
-      hipLaunchKernelGGL(outer_split_kernel, dim3((unsigned)tiles), dim3(256), 0, s, g);
-    else
-      hipLaunchKernelGGL(outer_update_kernel, dim3((unsigned)tiles), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(outer_update_kernel, dim3((unsigned)tiles), dim3(256), 0, s, g);
     NOISE_CHECK_LAUNCH();
   }
   return NOISE_OK;

@@ -321,24 +321,62 @@ def _strided(t):
 
 
 @pytest.mark.parametrize('n', [1, 31, 33, 100])
-def test_outer_update_on_split_operands(n):
-    """Enough 128 x 128 tiles for the bf16-split kernel (288 of them in one matrix), ragged outputs, padded and odd row
-    strides, a vector parameter, direction counts around its 32-direction chunks: against the fp64 sum. The split drops
-    terms below 2^-24 of a product and rounds 6 times per 32 directions (2^-23 allows for truncation inside an MFMA), and
-    w a is rounded once."""
+def test_outer_update_of_ragged_matrices(n):
+    """A matrix of more tiles than the GPU holds at once beside small ones, ragged outputs, padded and odd row strides, a
+    vector parameter, direction counts around the 32-direction chunks: against the fp64 sum. w a is rounded once and an
+    output adds n exact products in fp32, each addition rounding at most 2^-24 of what the magnitudes add up to (the
+    scale is a power of two)."""
     g = torch.Generator().manual_seed(41)
-    log_case(f'outer update, split operands, {n} directions')
+    log_case(f'outer update, ragged matrices, {n} directions')
     mats, w = _outer_case(g, [(4100, 1000, 0), (130, 257, 3), (0, 8, 0), (8, 32, 1), (1, 1, 0), (128, 128, 4)], n)
     for (a, b), got in zip(mats, _outer_gpu(mats, w, -0.25)):
         wa = (torch.ones(n, 1) if a is None else a).double() * w.double()[:, None]
         ref, mag = wa.t() @ b.double() * -0.25, wa.abs().t() @ b.double().abs() * 0.25
-        bound = (4 + 6 * (n // 32 + 1)) * 2 ** -23 * mag
-        assert ((got.double() - ref).abs() <= bound).all()
+        assert ((got.double() - ref).abs() <= (n + 2) * 2 ** -24 * mag).all()
+
+
+def test_outer_update_is_the_same_bits_alone_and_in_a_batch():
+    """A matrix's gradient depends neither on the matrices that share its launch nor on its position: 70 matrices, more
+    than one launch takes, with far more tiles than the GPU holds at once, against a call for each."""
+    g = torch.Generator().manual_seed(44)
+    n = 75
+    log_case('outer update, batch against single calls')
+    shapes = [(4100, 1000, 0), (512, 512, 0), (70, 130, 1), (0, 8, 0)] + [(64 + 7 * k, 96 + 3 * k, k % 4) for k in range(66)]
+    mats, w = _outer_case(g, shapes, n)
+    batch = _outer_gpu(mats, w, -0.3)
+    for k in (0, 1, 2, 3, 40, 63, 64, 69):
+        assert torch.equal(_outer_gpu(mats[k:k + 1], w, -0.3)[0], batch[k]), shapes[k]
+
+
+@pytest.mark.parametrize('scale_a', [2. ** -118, 2. ** 100])
+def test_outer_update_keeps_24_bits_of_operands_of_any_size(scale_a):
+    """Operands far from 1 have the same relative error as N(0, 1) ones, in an update of many tiles: the bound of
+    test_outer_update_of_ragged_matrices (every product and sum stays a normal fp32 number)."""
+    g = torch.Generator().manual_seed(45)
+    n = 40
+    log_case(f'outer update, operands of size {scale_a}')
+    mats, w = _outer_case(g, [(4100, 1000, 0)], n)
+    a, b = mats[0]
+    a, b = a.sign() * (0.5 + torch.rand(a.shape, generator=g)) * scale_a, b.sign() * (0.5 + torch.rand(b.shape, generator=g))
+    w = 0.5 + torch.rand(n, generator=g)
+    got = _outer_gpu([(a, b)], w, 1.0)[0]
+    wa = a.double() * w.double()[:, None]
+    ref, mag = wa.t() @ b.double(), wa.abs().t() @ b.double().abs()
+    assert ((got.double() - ref).abs() <= (n + 2) * 2 ** -24 * mag).all()
+
+
+def test_outer_update_of_nan_weights():
+    """z-score fitness of a population with one NaN loss makes every weight NaN: every gradient is NaN."""
+    g = torch.Generator().manual_seed(46)
+    log_case('outer update, NaN weights')
+    mats, w = _outer_case(g, [(4100, 1000, 0), (0, 8, 0), (70, 130, 1)], 64)
+    for got in _outer_gpu(mats, torch.full_like(w, float('nan')), -0.25):
+        assert torch.isnan(got).all()
 
 
 @pytest.mark.parametrize('pad,off', [(0, 1), (2, 0), (4, 3)])
 def test_outer_update_of_rows_off_16_byte_addresses(pad, off):
-    """Full 128 x 128 tiles whose rows start off 16-byte addresses (by the pointer, the row stride or both): the bits of
+    """Full tiles whose rows start off 16-byte addresses (by the pointer, the row stride or both): the bits of
     the aligned rows."""
     g = torch.Generator().manual_seed(43)
     log_case(f'outer update, row padding {pad}, offset {off}')
@@ -362,8 +400,8 @@ def test_outer_update_of_rows_off_16_byte_addresses(pad, off):
 
 
 def test_outer_update_of_non_finite_and_extreme_values():
-    """Infinities, NaN and values that bf16 would round to infinity: what the fp32 sum gives, in that column or row only;
-    tiny values (a product of 1e-30) keep their sum."""
+    """Infinities, NaN and values near fp32's largest: what the fp32 sum gives, in that column or row only; tiny values (a
+    product of 1e-30) keep their sum."""
     g = torch.Generator().manual_seed(42)
     n = 40
     log_case('outer update of non-finite and extreme values')
@@ -374,7 +412,7 @@ def test_outer_update_of_non_finite_and_extreme_values():
     b[3] = b[3].abs() + 0.1  # (no infinity times zero, and infinities of one sign per row)
     a[3, 5], a[3, 6], a[7, 2000], b[9, 700] = float('inf'), float('-inf'), float('nan'), float('inf')
     a[9] = a[9].abs() + 0.1
-    a[:, 17], a[3, 17] = 0, 3.4e38  # past bf16's largest; with b[3, 1] = 2^-100 finite
+    a[:, 17], a[3, 17] = 0, 3.4e38  # with b[3, 1] = 2^-100 finite
     b[3, 1] = 2 ** -100
     a[:, 4000] *= 1e-30
     got = _outer_gpu(mats, w, 1.0)[0]
