@@ -59,7 +59,7 @@ int outer_update_launch(const OuterUpdateArgs* mats, int n, const float* w, int 
 // Several tensors' Adam steps in one launch: up to ADAM_MAX tensors per launch, passed by value, with the running
 // total of ADAM_BLOCK-element blocks (block b belongs to the first tensor whose block_end exceeds b).
 constexpr int ADAM_MAX = 64;
-constexpr int ADAM_BLOCK = 2048;
+constexpr int ADAM_BLOCK = 512;
 struct AdamTensor {
   float* param;
   const float* grad;
@@ -68,12 +68,12 @@ struct AdamTensor {
   long n;
   float step_size;  // lr / (1 - beta1^step)
   float bc2_sqrt;   // sqrt(1 - beta2^step)
-  // set by the launch
-  int block_end;
-  int vec;          // the four pointers are 16-byte aligned
+  int block_end;    // set by the launch
 };
+template <int MAX>
 struct AdamBatchArgs {
-  AdamTensor t[ADAM_MAX];
+  static constexpr int MAX_TENSORS = MAX;
+  AdamTensor t[MAX];
   int n;
   float beta1, beta2, eps;
 };

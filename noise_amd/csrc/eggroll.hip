@@ -212,64 +212,43 @@ __global__ void __launch_bounds__(256, 2) outer_update_kernel(const OuterBatchAr
 }
 
 // torch.optim.AdamW (single-tensor path) with weight_decay = 0:
-// m = lerp(m, g, 1 - b1); v = b2 v + (1 - b2) g^2; p -= (lr / bc1) m / (sqrt(v) / sqrt(bc2) + eps).
-struct AdamConst {
-  float step_size, bc2_sqrt, beta1, beta2, eps;
-};
-__device__ __forceinline__ void adam_element(float& param, float gr, float& m, float& v, const AdamConst& c) {
-  // the fused operations are written out, so that the vector and the scalar path round alike
-  const float w = 1.f - c.beta1, d = gr - m;
-  m = w < 0.5f ? fmaf(w, d, m) : fmaf(-(1.f - w), d, gr);
-  v = fmaf(gr, (1.f - c.beta2) * gr, c.beta2 * v);
-  const float denom = sqrtf(v) / c.bc2_sqrt + c.eps;
-  param = fmaf(-c.step_size, m / denom, param);
-}
+// m = lerp(m, g, 1 - b1); v = b2 v + (1 - b2) g^2; p -= (lr / bc1) m / (sqrt(v) / sqrt(bc2) + eps), the fused operations
+// written out.
 // Every tensor of an optimizer step in one launch: block b serves the tensor whose range of ADAM_BLOCK-element blocks
-// holds it (a binary search over the running totals). Bound by HBM, 28 bytes per element. Four elements per thread and
-// access where the tensor's four pointers allow 16-byte vectors, two of them in flight before any is used: 37.7M
-// parameters 497 us (2.1 TB/s) with one element per thread -> 176 us
-// (6.0 TB/s).
-__global__ void __launch_bounds__(256) adam_batch_kernel(const AdamBatchArgs g) {
+// holds it (a binary search over the running totals; a linear scan took 481 us for the model's tensors). Bound by HBM, 28
+// bytes per element. Two elements per thread, every load before the first store: the model's 61 tensors 190 us (5.6 TB/s),
+// 37.7M parameters in one tensor 181, off 16-byte addresses 187. (One element per thread 202, 173 and 187; blocks of 2048
+// elements in 16-byte vectors 200, 198 and 228, and 5.4 against 4.5 for 100,000 elements.)
+// MAX: tensors the arguments hold; one tensor's launch copies 64 bytes of them instead of 3.6 KiB.
+template <int MAX>
+__global__ void __launch_bounds__(256) adam_batch_kernel(const AdamBatchArgs<MAX> g) {
+  constexpr int V = ADAM_BLOCK / 256;
   const long b = blockIdx.x;
-  int lo = 0, hi = g.n - 1;
+  int lo = 0, hi = MAX > 1 ? g.n - 1 : 0;
   while (lo < hi) {
     const int mid = (lo + hi) >> 1;
     if (b < g.t[mid].block_end) hi = mid;
     else lo = mid + 1;
   }
   const AdamTensor& t = g.t[lo];
-  const AdamConst c{t.step_size, t.bc2_sqrt, g.beta1, g.beta2, g.eps};
-  const long base = (b - (lo ? g.t[lo - 1].block_end : 0)) * ADAM_BLOCK;
-  if (t.vec && base + ADAM_BLOCK <= t.n) {
-    constexpr int V = ADAM_BLOCK / 1024;
-    float4 p4[V], g4[V], m4[V], v4[V];
+  const long i0 = (b - (lo ? g.t[lo - 1].block_end : 0)) * ADAM_BLOCK + threadIdx.x;
+  const float w = 1.f - g.beta1;
+  float p[V], gr[V], m[V], v[V];
 #pragma unroll
-    for (int q = 0; q < V; ++q) {
-      const long i = base + 1024 * q + 4 * threadIdx.x;
-      p4[q] = *reinterpret_cast<const float4*>(t.param + i);
-      g4[q] = *reinterpret_cast<const float4*>(t.grad + i);
-      m4[q] = *reinterpret_cast<const float4*>(t.m + i);
-      v4[q] = *reinterpret_cast<const float4*>(t.v + i);
-    }
-#pragma unroll
-    for (int q = 0; q < V; ++q) {
-      const long i = base + 1024 * q + 4 * threadIdx.x;
-      adam_element(p4[q].x, g4[q].x, m4[q].x, v4[q].x, c);
-      adam_element(p4[q].y, g4[q].y, m4[q].y, v4[q].y, c);
-      adam_element(p4[q].z, g4[q].z, m4[q].z, v4[q].z, c);
-      adam_element(p4[q].w, g4[q].w, m4[q].w, v4[q].w, c);
-      *reinterpret_cast<float4*>(t.param + i) = p4[q];
-      *reinterpret_cast<float4*>(t.m + i) = m4[q];
-      *reinterpret_cast<float4*>(t.v + i) = v4[q];
-    }
-    return;
+  for (int q = 0; q < V; ++q) {
+    const long i = i0 + 256 * q;
+    if (i < t.n) p[q] = t.param[i], gr[q] = t.grad[i], m[q] = t.m[i], v[q] = t.v[i];
   }
-  for (long i = base + threadIdx.x; i < min(base + ADAM_BLOCK, t.n); i += 256) {
-    float p = t.param[i], m = t.m[i], v = t.v[i];
-    adam_element(p, t.grad[i], m, v, c);
-    t.param[i] = p;
-    t.m[i] = m;
-    t.v[i] = v;
+#pragma unroll
+  for (int q = 0; q < V; ++q) {
+    const long i = i0 + 256 * q;
+    if (i >= t.n) return;
+    const float d = gr[q] - m[q];
+    m[q] = w < 0.5f ? fmaf(w, d, m[q]) : fmaf(-(1.f - w), d, gr[q]);
+    v[q] = fmaf(gr[q], (1.f - g.beta2) * gr[q], g.beta2 * v[q]);
+    t.m[i] = m[q];
+    t.v[i] = v[q];
+    t.param[i] = fmaf(-t.step_size, m[q] / (sqrtf(v[q]) / t.bc2_sqrt + g.eps), p[q]);
   }
 }
 
@@ -370,18 +349,20 @@ int adam_batch_launch(const AdamTensor* tensors, int n, float beta1, float beta2
     }
     if (blocks > 0x7fffffffL) return NOISE_ENOTSUP;
   }
-  for (int base = 0; base < n; base += ADAM_MAX) {
-    AdamBatchArgs g{};
-    g.n = std::min(ADAM_MAX, n - base);
+  auto launch = [&](auto g, int base, int count) {
+    g.n = count;
     g.beta1 = beta1, g.beta2 = beta2, g.eps = eps;
     long blocks = 0;
-    for (int k = 0; k < g.n; ++k) {
-      AdamTensor& t = g.t[k] = tensors[base + k];
-      t.vec = !(((uintptr_t)t.param | (uintptr_t)t.grad | (uintptr_t)t.m | (uintptr_t)t.v) & 15);
-      blocks += (t.n + ADAM_BLOCK - 1) / ADAM_BLOCK;
-      t.block_end = (int)blocks;
+    for (int k = 0; k < count; ++k) {
+      g.t[k] = tensors[base + k];
+      blocks += (g.t[k].n + ADAM_BLOCK - 1) / ADAM_BLOCK;
+      g.t[k].block_end = (int)blocks;
     }
-    hipLaunchKernelGGL(adam_batch_kernel, dim3((unsigned)blocks), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(adam_batch_kernel<decltype(g)::MAX_TENSORS>, dim3((unsigned)blocks), dim3(256), 0, s, g);
+  };
+  for (int base = 0; base < n; base += ADAM_MAX) {
+    if (n == 1) launch(AdamBatchArgs<1>{}, base, 1);
+    else launch(AdamBatchArgs<ADAM_MAX>{}, base, std::min(ADAM_MAX, n - base));
     NOISE_CHECK_LAUNCH();
   }
   return NOISE_OK;

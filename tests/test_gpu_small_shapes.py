@@ -185,12 +185,12 @@ def test_attention_of_64_and_128_queries_per_workgroup_agree_bit_for_bit(T, wind
     assert torch.isfinite(alone[0].float()).all()
 
 
-def test_adam_vector_and_scalar_elements_agree():
-    """Tensors of whole and ragged blocks, at 16-byte addresses (four elements per access) and one element off (scalar):
-    the same bits, and nothing written past the end."""
+def test_adam_of_whole_and_ragged_blocks_at_any_address():
+    """Tensors of whole and ragged blocks, at 16-byte addresses and one element off: the same bits, and nothing written
+    past the end."""
     import math
     g = torch.Generator().manual_seed(37)
-    for n in (1, 2047, 2048, 2049, 3 * 2048 + 1023):
+    for n in (1, 255, 257, 511, 513, 2047, 2048, 2049, 3 * 2048 + 1023):
         log_case(f'adam n={n}')
         vals = [torch.randn(n, generator=g), torch.randn(n, generator=g), torch.randn(n, generator=g),
                 torch.rand(n, generator=g)]
@@ -207,6 +207,36 @@ def test_adam_vector_and_scalar_elements_agree():
             res.append((p.clone(), m.clone(), v.clone()))
         for x, y in zip(*res):
             assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize('count', [1, 2, 64, 65, 129])
+def test_adam_batch_is_each_tensor_alone(count):
+    """Batches of one tensor, of several, of as many as one launch takes and of more: every tensor gets the bits of a call
+    of its own, with its own step size, and no other element of the flat buffers changes."""
+    g = torch.Generator().manual_seed(47)
+    log_case(f'adam batch of {count}')
+    sizes = [(1, 511, 256, 513, 1000, 512)[k % 6] for k in range(count)]
+    total = sum(sizes) + 3 * count
+    start = [torch.randn(total, generator=g) for _ in range(3)] + [torch.rand(total, generator=g)]
+    batch, single = ([t.to(DEV) for t in start] for _ in range(2))
+
+    def items(bufs):
+        at, out = 0, []
+        for k, n in enumerate(sizes):
+            out.append((*(t.data_ptr() + 4 * at for t in bufs), n, 1e-3 / (k + 1), 0.2 + 0.001 * k))
+            at += n + 3
+        return out
+    ptr, c, _keep = _lib.adam_tensors(items(batch))
+    _lib.call('noise_adam_batch', ptr, c, 0.5, 0.95, 1e-8, _stream())
+    for p, gr, m, v, n, step, bc2 in items(single):
+        _lib.call('noise_adam', p, gr, m, v, n, step, 0.5, 0.95, 1e-8, bc2, _stream())
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, y) for x, y in zip(batch, single))
+    at = 0
+    for n in sizes:
+        for t, before in zip(batch, start):
+            assert torch.equal(t[at + n:at + n + 3].cpu(), before[at + n:at + n + 3])
+        at += n + 3
 
 
 @pytest.mark.parametrize('pairs', [2, 15, 16, 17, 2047, 2049])
