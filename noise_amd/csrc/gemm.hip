@@ -668,11 +668,12 @@ __global__ void __launch_bounds__(256) weight_tiles_kernel(const bf16* __restric
 // member reads the same x, four rows against four directions (an antithetic pair's two members share the dot): each b
 // is read once per four rows and each x row once per four directions instead of both for every dot. Bound by the traffic
 // out of L2: 256 members (128 pairs) x 2048 tokens on one x 81.5 us with a wave per row, 27.1 now
-// with the weight copy (5.5) in the same launch. A lane adds its 8
-// columns in order and the lanes' sums meet in one tree, whatever the grouping.
-template <int DB>
+// with the weight copy (5.5) in the same launch. Rows of their own deeper than one step of 512 columns keep a wave each
+// (RB = 1): grouped, a quarter of the waves walk the steps, each behind the loads of four rows (65,536 rows of 2048 columns
+// 56.2 us against 48.7, 24,576 21.7 against 15.5). One direction on a shared x takes the rows as one member's. A lane adds
+// its 8 columns in order and the lanes' sums meet in one tree, whatever the grouping.
+template <int RB, int DB>
 __device__ __forceinline__ void rowdot_units(const RowdotArgs& g, int wave, int nwaves) {
-  constexpr int RB = 4;
   const int lane = threadIdx.x & 63;
   const int members = g.M / g.T, dirs = (members + (1 << g.pair_shift) - 1) >> g.pair_shift;
   const int rt = (g.T + RB - 1) / RB, units = rt * (DB == 1 ? members : (dirs + DB - 1) / DB);
@@ -723,27 +724,29 @@ __device__ __forceinline__ void rowdot_units(const RowdotArgs& g, int wave, int 
   }
 }
 // Workgroups 0 .. tile_blocks - 1 copy w into WTILE, the others take the row dots.
-template <int DB>
+template <int RB, int DB>
 __global__ void __launch_bounds__(256) rowdot_kernel(RowdotArgs g, int tile_blocks, const bf16* __restrict__ w, int K2,
                                                      long chunks, bf16* __restrict__ out) {
   const int b = blockIdx.x - tile_blocks;
   if (b < 0)
     weight_tile_chunk(w, K2, K2, chunks, out, (long)blockIdx.x * 256 + threadIdx.x);
   else
-    rowdot_units<DB>(g, b * 4 + (threadIdx.x >> 6), (gridDim.x - tile_blocks) * 4);
+    rowdot_units<RB, DB>(g, b * 4 + (threadIdx.x >> 6), (gridDim.x - tile_blocks) * 4);
 }
 int rowdot_any(const RowdotArgs& g, int tile_blocks, const bf16* w, int K2, long chunks, bf16* out, hipStream_t stream) {
   if (!g.x || !g.b || !g.u || g.M <= 0 || g.K <= 0 || g.K % 8 || g.ldx % 8 || g.x_mstride % 8 || g.ldb % 4 || g.T <= 0 ||
       g.M % g.T)
     return NOISE_EINVAL;
-  const int members = g.M / g.T, dirs = (members + (1 << g.pair_shift) - 1) >> g.pair_shift, rt = (g.T + 3) / 4;
-  const bool shared = g.x_mstride == 0 && members > 1;
-  const long units = (long)rt * (shared ? (dirs + 3) / 4 : members);
+  const int members = g.M / g.T, dirs = (members + (1 << g.pair_shift) - 1) >> g.pair_shift;
+  const bool shared = g.x_mstride == 0 && dirs > 1, deep = !shared && g.K > 512;
+  const long units = (long)(deep ? g.T : (g.T + 3) / 4) * (shared ? (dirs + 3) / 4 : members);
   const unsigned grid = (unsigned)(tile_blocks + std::min<long>((units + 3) / 4, 8192));
-  if (shared)
-    hipLaunchKernelGGL(rowdot_kernel<4>, dim3(grid), dim3(256), 0, stream, g, tile_blocks, w, K2, chunks, out);
-  else
-    hipLaunchKernelGGL(rowdot_kernel<1>, dim3(grid), dim3(256), 0, stream, g, tile_blocks, w, K2, chunks, out);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, g, tile_blocks, w, K2, chunks, out);
+  };
+  if (shared) launch(rowdot_kernel<4, 4>);
+  else if (deep) launch(rowdot_kernel<1, 1>);
+  else launch(rowdot_kernel<4, 1>);
   NOISE_CHECK_LAUNCH();
   return NOISE_OK;
 }

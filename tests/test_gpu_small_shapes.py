@@ -106,12 +106,14 @@ def test_tile_configurations_of_the_head_agree_bit_for_bit(head, T):
 
 @pytest.mark.parametrize('shared', ['q', 'k'])
 @pytest.mark.parametrize('qk_norm', [0, 1])
-def test_attention_on_shared_heads_equals_packed_rows(shared, qk_norm):
+@pytest.mark.parametrize('n', [3, 40])
+def test_attention_on_shared_heads_equals_packed_rows(n, shared, qk_norm):
     """Attention on separate operands, one of q and k and the values stored once per batch row for every draw, is bit for
-    bit the attention on packed q | k | v rows that hold a copy per member."""
+    bit the attention on packed q | k | v rows that hold a copy per member: 64 queries per workgroup (3 draws) and 128
+    (40)."""
     g = torch.Generator().manual_seed(34)
-    n, b, T, window = 3, 2, 256, 100
-    log_case(f'attention on shared heads: {shared} shared, qk_norm={qk_norm}')
+    b, T, window = 2, 256, 100
+    log_case(f'attention on shared heads: {n} draws, {shared} shared, qk_norm={qk_norm}')
 
     def heads(blocks):
         x = torch.randn(blocks * T, 8, 64, generator=g)
@@ -530,8 +532,8 @@ def test_scores_of_a_credit_chunk_equal_those_of_its_outputs(kind, n, b, T, wind
 @pytest.mark.parametrize('members,T,pair', [(1, 1, 0), (2, 7, 1), (5, 33, 1), (9, 130, 0), (18, 4, 1)])
 @pytest.mark.parametrize('din', [64, 512, 1088])
 def test_linear_on_shared_activations_equals_separate_copies(members, T, pair, din):
-    """The input-side dots take four rows against one direction, or against four where members share one activation:
-    the same bits, for ragged row and direction groups, odd member counts and pairs."""
+    """The input-side dots take four rows (deeper than 512 columns: one) against one direction, or four against four where
+    members share one activation: the same bits, for ragged row and direction groups, odd member counts and pairs."""
     from noise_amd import ops
     g = torch.Generator(DEV).manual_seed(46)
     log_case(f'linear on shared activations members={members} T={T} pair={pair} din={din}')
