@@ -60,6 +60,9 @@ struct Cfg {
   static constexpr int STAGE = (BM + BN) * BK;   // bf16 elements per LDS stage
   // threads summing one row's x.b partials: two halves at most, so that every configuration adds them in one order
   static constexpr int UGROUPS = NTH / BM < 2 ? NTH / BM : 2;
+  // every thread has such a half: known here, so that the large tiles carry no test of it (as runtime tests, and with a
+  // bound of its own for every epilogue's last tiled rows, their epilogues took 1.5-5% longer)
+  static constexpr bool ALL_U = UGROUPS * BM == NTH;
   static_assert(BK == 32 || BK == 64, "BK must be 32 or 64");
   static_assert(WM % 16 == 0 && WN % 16 == 0 && FN % 2 == 0, "wave tile must be a multiple of 16 x 32");
   static_assert(LA * ROWS_PER_DMA * NW == BM && LB * ROWS_PER_DMA * NW == BN, "DMA must tile evenly");
@@ -153,7 +156,12 @@ lowrank_gemm_kernel(const LowrankGemmArgs g) {
     for (int d = 0; d < C::LA; ++d) {
       if (g.a_tiled) {
         // the 16 rows of this instruction are one 1 KiB TILE16 tile per 32-deep stage
-        const int G = min((m0 >> 4) + wave * C::LA + d, (g.M - 1) >> 4);
+        // (only the fp16 head's operand may end in a partial group)
+        int G;
+        if constexpr (EPI == EPI_CE_F16)
+          G = min(m0 + (wave * C::LA + d) * C::ROWS_PER_DMA, (g.M - 1) & ~15) >> 4;
+        else
+          G = min(m0 + (wave * C::LA + d) * C::ROWS_PER_DMA, g.M - 16) >> 4;
         a_src[d] = (long)G * 16 * g.lda + 8 * lane;
       } else {
         const int r = (wave * C::LA + d) * C::ROWS_PER_DMA + lrow;
@@ -236,7 +244,7 @@ lowrank_gemm_kernel(const LowrankGemmArgs g) {
     if (F16 && tid < BN / 4) pre_sc = *reinterpret_cast<const float4*>(g.col_scale + n0 + 4 * tid);
     if (tid == 0) pre_sign = pfirst == plast ? g.sign[pfirst] : 0.f;
     const int row = min(m0 + tid % BM, g.M - 1), grp = tid / BM;
-    if (grp < C::UGROUPS) {
+    if (C::ALL_U || grp < C::UGROUPS) {
       const int q0 = grp * g.u_parts / C::UGROUPS, q1 = (grp + 1) * g.u_parts / C::UGROUPS;
       const float* up = g.u + (long)row * g.u_ld + (long)seg * g.u_parts * g.u_qstride;
       float u = 0.f;
@@ -266,7 +274,7 @@ lowrank_gemm_kernel(const LowrankGemmArgs g) {
       if (tid < BN / 4) *reinterpret_cast<float4*>(&ep_a[4 * tid]) = pre_ab;
     }
     if (tid == 0) ep_sign = pre_sign;
-    if (tid < C::UGROUPS * BM) ep_u[tid / BM][tid % BM] = pre_u;
+    if (C::ALL_U || tid < C::UGROUPS * BM) ep_u[tid / BM][tid % BM] = pre_u;
     if (CE && tid < BM) ep_t[tid] = pre_t;
   };
 
