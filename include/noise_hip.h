@@ -280,6 +280,18 @@ int noise_ac_qkv(void* qkv, const void* rot_cos, const void* rot_sin, const floa
 int noise_norm_dot(const float* x, void* h, const float* b, float* u, const float* sign, int members, int T,
                    int pair_shift, const noise_pending_t* pend, int npend, noise_stream_t stream);
 
+/* The output tile that the tile GEMM takes for a product of `rows` rows over `in` into `out` columns (in % 64 == 0, out %
+ * 128 == 0), or NOISE_EINVAL: the choice is by time alone, every tile gives the same bits. The head's `in` is 512
+ * (NOISE_HEAD_BF16), 1024 (NOISE_HEAD_FP32) or 1536 (NOISE_HEAD_FP32_SPLIT). */
+#define NOISE_RESULT_BF16 0
+#define NOISE_RESULT_F32 1  /* written or accumulated */
+#define NOISE_RESULT_HEAD 2 /* noise_head_ce */
+#define NOISE_TILE_256X256 0
+#define NOISE_TILE_256X128 1
+#define NOISE_TILE_128X128 2
+#define NOISE_TILE_64X64 3
+int noise_gemm_tile(int rows, int in, int out, int result);
+
 /* hidden = bf16(relu(lowrank(h, w_fc))^2) [members*T, f] in hidden_layout (NOISE_LAYOUT_ROWS or
  * NOISE_LAYOUT_TILE16, the layout noise_dense_bf16 loads fastest) and its dot partials with bf16(b_proj),
  * part-major: upart [noise_mlp_fc_parts(f), members*T] (one partial per 256 columns), for the

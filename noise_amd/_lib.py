@@ -21,6 +21,8 @@ QK_BF16, QK_F16, QK_F16_Q_LOG2, QK_BF16_V_BF16 = 0, 1, 2, 3
 LAYOUT_ROWS, LAYOUT_TILE16, LAYOUT_WTILE = 0, 1, 2
 CE_MEMBER_MEAN, CE_NONE, CE_SUM, CE_MEAN = 0, 1, 2, 3
 HEAD_BF16, HEAD_FP32_SPLIT, HEAD_FP32 = 0, 1, 2  # noise_head_ce's weight formats (NOISE_HEAD_*)
+RESULT_BF16, RESULT_F32, RESULT_HEAD = 0, 1, 2  # noise_gemm_tile's results and tiles
+TILE_256X256, TILE_256X128, TILE_128X128, TILE_64X64 = 0, 1, 2, 3
 
 # name -> argtypes in declaration order; every entry point returns int. Pointers (device buffers,
 # the stream) are c_void_p.
@@ -46,6 +48,7 @@ SIGNATURES = {
     'noise_weight_tiles': [P, I, I, P, P],
     'noise_dense_bf16': [P, I, I, I, P, I, I, I, P, P],
     'noise_mlp_fc_parts': [I],
+    'noise_gemm_tile': [I, I, I, I],
     'noise_mlp_fc': [P, P, I, I, P, P, P, P, I, I, I, P, I, P, P],
     'noise_head_ce_workspace_size': [I, I, I, I, SP],
     'noise_head_ce': [P, I, P, P, I, I, P, P, P, P, L, I, I, I, I, P, P, P, S, P, I, P],
@@ -173,7 +176,7 @@ def pending(*items):
 
 
 # Entry points whose int result is a value, not a status.
-VALUE_RESULT = {'noise_version', 'noise_mlp_fc_parts'}
+VALUE_RESULT = {'noise_version', 'noise_mlp_fc_parts', 'noise_gemm_tile'}
 
 _lib = None
 

@@ -476,6 +476,8 @@ int noise_dense_bf16(const void* x, int x_layout, int in, int out, const void* w
   return lowrank_gemm_launch(EPI_DENSE, g, static_cast<hipStream_t>(stream));
 }
 
+int noise_gemm_tile(int rows, int in, int out, int result) { return lowrank_gemm_tile(rows, out, in, result); }
+
 int noise_mlp_fc_parts(int f) { return xs_relu2_parts(f); }
 
 int noise_mlp_fc(const void* h, const void* w_fc, int d, int f, const float* a_fc, const float* u,

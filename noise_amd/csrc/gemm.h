@@ -135,6 +135,8 @@ int head_weight_f16_launch(const float* w, long ldw, const float* gain, int N, i
 
 // Number of per-row partials EPI_CE writes for an N-column output (0: N unsupported).
 int lowrank_gemm_parts(int N);
+// The tile (NOISE_TILE_*) of an M x N product over K whose epilogue writes `result` (NOISE_RESULT_*), or NOISE_EINVAL.
+int lowrank_gemm_tile(int M, int N, int K, int result);
 int lowrank_gemm_launch(int epi, const LowrankGemmArgs& g, hipStream_t stream);
 
 // The weight-resident K = 512 relu^2 GEMM (gemm_xs.hip): partials per row it writes for N columns (0: N

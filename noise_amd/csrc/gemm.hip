@@ -619,33 +619,47 @@ int launch_cfg(const LowrankGemmArgs& g, hipStream_t stream) {
 
 bool use_big(int N) { return N % 256 == 0; }
 
-// The configuration of a launch, by how its tiles fill the CUs. Every configuration contracts K in the same order and
-// rounds alike, so the choice never changes a result.
-//  - 64 x 64 tiles while at most three of them fall on a CU: a larger tile then leaves most CUs idle behind one long K
-//    chain (2048 x 512 outputs, K = 2048: 42.9 us on 16 tiles of 256 x 256, 20.9 on 64 of 128 x 128, 10.7 on 256 of
-//    64 x 64; 6144 rows, three per CU: 43.4, 22.2, 20.4; 8192 rows, four per CU: 43.7, 23.3, 25.9). Its steps are bound by
-//    their own chain (LDS reads, MFMAs: 164 ns each), not by loads in flight or barriers: rings of 6 and 8 stages instead
-//    of 4 took 11.5 and 11.2 us against 10.5 in those 256 tiles, 8 stages opened two at a time 10.9.
-//  - beyond that, the fewer rounds of the GPU. In units of one round of 256 x 256 tiles (one workgroup per CU, 55.7 us
-//    at K = 2048), 128 x 128 tiles, two workgroups per CU, cost 0.585 a full round and 0.36 where the last one leaves
-//    one per CU; 256 x 128 tiles (N not a multiple of 256) 0.56. So 128 x 128 tiles run ragged ends (16384 rows: 47.4
-//    -> 34.7 us; 38400: 152 -> 134) and 256 x 256 ones every large launch (65536 rows: 146 against 118 us).
+// What an epilogue writes (NOISE_RESULT_*).
+enum class Result { BF16, F32, HEAD };
+
+// The configuration of a launch: the least time by a model of its rounds of the GPU. Every configuration contracts K in
+// the same order and rounds alike, so the choice never changes a result.
+// A round (one workgroup per CU of 256 x 256 or 256 x 128 tiles; two of 128 x 128, or one where the last round has no more;
+// four of 64 x 64, or one to three) takes a part that grows with K and an epilogue that does not. The constants, in us,
+// are fitted to 1856 calls measured with every configuration (dense and low-rank products from row-major and tiled
+// operands at K = 64 .. 2048 into 384, 512 and 2048 columns, the head's formats over 256 .. 8192, 16 .. 4096 128 x 128 tiles
+// each); the choice is on average 0.3 to 1% behind the fastest of the four by kind of call. The smaller tiles have to be
+// 8% ahead, so that no call measured more than 5% slower than on the large tiles alone. Per 1000 of K a large tile is the
+// cheaper one by operand traffic, but a round of it cannot be shared: c_proj of 2048 rows (K = 2048, 512 columns) runs 42.9
+// us on 16 tiles of 256 x 256, 20.9 on 64 of 128 x 128 and 10.7 on 256 of 64 x 64; of 6144 rows 46.4, 23.2 and 26.8; 20,000
+// rows into 2048 columns 160, 194 and 354. A 64 x 64 tile's steps are bound by their own chain (LDS reads, MFMAs: 164 ns
+// each), not by loads in flight or barriers: rings of 6 and 8 stages instead of 4 took 11.5 and 11.2 us against 10.5 in
+// those 256 tiles, 8 stages opened two at a time 10.9.
 enum class Tile { BIG, WIDE, MID, SMALL };
-Tile pick_tile(int M, int N) {
+Tile pick_tile(int M, int N, int K, Result result) {
   const long cus = num_cus();
   const auto tiles = [&](long bm, long bn) { return (M + bm - 1) / bm * ((N + bn - 1) / bn); };
-  if (tiles(64, 64) <= 3 * cus) return Tile::SMALL;
-  const long mid = tiles(128, 128), rest = mid % (2 * cus);
-  const double mid_cost = mid / (2 * cus) * 0.585 + (rest > cus ? 0.585 : rest ? 0.36 : 0.);
-  const long wide = tiles(256, use_big(N) ? 256 : 128);
-  const double cost = (wide + cus - 1) / cus * (use_big(N) ? 1. : 0.56);
-  return mid_cost < cost ? Tile::MID : use_big(N) ? Tile::BIG : Tile::WIDE;
+  // epilogue of a 256 x 256 round: bf16 results, fp32 ones (twice the stores, or read and written), capped logits
+  const double e = result == Result::BF16 ? 7.4 : result == Result::F32 ? 17. : 35., k = K * 1e-3;
+  const double rounds = (double)((tiles(256, use_big(N) ? 256 : 128) + cus - 1) / cus);
+  const double large = rounds * (use_big(N) ? e + 22.7 * k : 0.46 * e + 15. * k);
+  const long m = tiles(128, 128), mr = m % (2 * cus);
+  double mid = (double)(m / (2 * cus) + (mr > cus)) * (0.34 * e + 16.9 * k);
+  if (mr > 0 && mr <= cus) mid += 0.26 * e + 6.4 * k;
+  if (result == Result::HEAD) mid *= 1.2;
+  const long s = tiles(64, 64), sr = (s % (4 * cus) + cus - 1) / cus;
+  const double small = (double)(s / (4 * cus)) * (0.15 * e + 17.5 * k) + (double)sr * (0.042 * e + 2.5 * k);
+  if (small <= mid && small < 0.92 * large) return Tile::SMALL;
+  if (mid < 0.92 * large) return Tile::MID;
+  return use_big(N) ? Tile::BIG : Tile::WIDE;
 }
 
 template <int EPI>
 int launch_epi(const LowrankGemmArgs& g, hipStream_t stream) {
+  constexpr bool HEAD = EPI == EPI_CE || EPI == EPI_CE_F16;
+  const Result result = HEAD ? Result::HEAD : EPI == EPI_RESID || g.out_f32 ? Result::F32 : Result::BF16;
   // (EPI_QKV serves token counts that are no multiple of 32: one configuration per width)
-  const Tile t = EPI == EPI_QKV ? (use_big(g.N) ? Tile::BIG : Tile::WIDE) : pick_tile(g.M, g.N);
+  const Tile t = EPI == EPI_QKV ? (use_big(g.N) ? Tile::BIG : Tile::WIDE) : pick_tile(g.M, g.N, g.K, result);
   if constexpr (EPI != EPI_QKV) {
     if (t == Tile::SMALL) return launch_cfg<CFG_SMALL, EPI>(g, stream);
     if (t == Tile::MID) return launch_cfg<CFG_MID, EPI>(g, stream);
@@ -839,6 +853,11 @@ int head_weight_f16_launch(const float* w, long ldw, const float* gain, int N, i
                      tiled, reinterpret_cast<_Float16*>(out), scale);
   NOISE_CHECK_LAUNCH();
   return NOISE_OK;
+}
+
+int lowrank_gemm_tile(int M, int N, int K, int result) {
+  if (M <= 0 || N <= 0 || K <= 0 || N % 128 || K % 64 || result < 0 || result > 2) return NOISE_EINVAL;
+  return (int)pick_tile(M, N, K, (Result)result);
 }
 
 int lowrank_gemm_parts(int N) {
