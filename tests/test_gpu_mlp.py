@@ -101,7 +101,8 @@ def test_lowrank_linear_ragged_rows(T):
 
 @pytest.mark.parametrize('dout', [384, 640])
 def test_lowrank_linear_narrow_tiles(dout):
-    """Output widths that are a multiple of 128 but not of 256 run the tile GEMM's 256 x 128 configuration."""
+    """Output widths that are a multiple of 128 but not of 256, in a launch of few rows (the tile GEMM's 64 x 64 tiles; its
+    larger ones in test_gpu_small_shapes.py)."""
     from noise_amd import ops
     g = torch.Generator().manual_seed(6)
     P, T, din = 4, 128, 512
@@ -119,8 +120,8 @@ def test_lowrank_linear_narrow_tiles(dout):
 
 @pytest.mark.parametrize('dout,din', [(384, 2048), (640, 1024)])
 def test_dense_wtile_weight_on_narrow_tiles(dout, din):
-    """The dense c_proj product with a WTILE weight on the 256 x 128 tile configuration (output widths a multiple of
-    128, not of 256) returns exactly the row-major weight's result, and bf16(x W^T) within one bf16 step."""
+    """The dense c_proj product with a WTILE weight and an output width that is a multiple of 128, not of 256, in a launch
+    of few rows (64 x 64 tiles) returns exactly the row-major weight's result, and bf16(x W^T) within one bf16 step."""
     from noise_amd import _lib
     g = torch.Generator().manual_seed(8)
     P, T = 2, 128
@@ -188,7 +189,7 @@ def test_dense_block_counts_around_the_steady_loop(P):
 def test_dense_tile_gemm_depths_around_the_steady_loop(din):
     """The tile GEMM's dense product runs k stages 1 .. KT - 4 (KT = din / 32) from its steady loop in pairs: none at
     KT = 4 or 6, one pair at 8, one at 10 (an odd count left for the general loop), 22 at 48. bf16(x W^T) within one
-    bf16 step everywhere."""
+    bf16 step everywhere. 1024 rows: 64 x 64 tiles (the others in test_gpu_small_shapes.py)."""
     from noise_amd import _lib
     P, T, dout = 4, 256, 512
     M = P * T

@@ -45,17 +45,31 @@ def test_weight_resident_product_from_both_weight_layouts(members, T, dout):
     assert ((rows.cpu().double() - ref).abs() <= bound).all()
 
 
+def _members_on_tiles(T, din, dout, result, most=140000):
+    """tile -> the fewest members of T rows whose product takes it, for every tile that the rule takes up to `most`
+    rows."""
+    out = {}
+    for m in range(1, most // T + 1):
+        out.setdefault(_lib.value('noise_gemm_tile', m * T, din, dout, result), m)
+    return out
+
+
 @pytest.mark.parametrize('out', ['f32', 'bf16', 'accumulate'])
-@pytest.mark.parametrize('dout,din,T', [(512, 576, 1000), (640, 128, 1000), (512, 2048, 250)])
+@pytest.mark.parametrize('dout,din,T', [(512, 576, 1000), (640, 1088, 1000), (512, 2048, 250), (384, 2048, 250)])
 def test_tile_configurations_of_the_linear_agree_bit_for_bit(dout, din, T, out):
-    """The tile GEMM takes 64 x 64, 128 x 128 or the large tiles by the number of rows. Every member's rows are the same
-    bits whichever it takes: 48,000 rows (256 x 256 or, at 640 columns, 256 x 128 tiles), the first quarter of them
-    (128 x 128), and slices of up to 5,000 rows down to one member (64 x 64). T = 1000 and 250 leave ragged last tiles
-    and tiles that straddle members."""
+    """The tile GEMM takes 64 x 64, 128 x 128 or the large tiles (256 x 256; 256 x 128 where the columns are no multiple
+    of 256) by the shape. Every member's rows are the same bits whichever it takes: the fewest rows that take each
+    tile, against a few members on 64 x 64 tiles. T = 1000 and 250 leave ragged last tiles and tiles that straddle
+    members."""
     from noise_amd import ops
+    result = _lib.RESULT_BF16 if out == 'bf16' else _lib.RESULT_F32
+    on = _members_on_tiles(T, din, dout, result)
+    large = _lib.TILE_256X128 if dout % 256 else _lib.TILE_256X256
+    assert set(on) == {large, _lib.TILE_128X128, _lib.TILE_64X64} and on[_lib.TILE_64X64] == 1
     g = torch.Generator().manual_seed(32)
-    P = 48000 // T
-    log_case(f'linear tile configurations {din}->{dout} T={T} {out}')
+    P, few = max(on.values()), max(1, 1000 // T)
+    assert _lib.value('noise_gemm_tile', few * T, din, dout, result) == _lib.TILE_64X64
+    log_case(f'linear tile configurations {din}->{dout} T={T} {out}: members {on}')
     x = torch.randn(P, T, din, generator=g).bfloat16().to(DEV)
     w = (torch.randn(dout, din, generator=g) * din ** -0.5).bfloat16().to(DEV)
     a, b = torch.randn(P, dout, generator=g).to(DEV), torch.randn(P, din, generator=g).to(DEV)
@@ -66,20 +80,63 @@ def test_tile_configurations_of_the_linear_agree_bit_for_bit(dout, din, T, out):
         kw = dict(out=res[lo:hi].clone(), accumulate=True) if out == 'accumulate' else \
             dict(out_dtype=torch.bfloat16 if out == 'bf16' else torch.float32)
         return ops.lowrank_linear(x[lo:hi], w, a[lo:hi], b[lo:hi], sign[lo:hi], **kw)
-    whole = run(0, P)
-    for lo, hi in ((0, P // 4), (1, 1 + 5000 // T), (P - 1, P)):
-        assert torch.equal(run(lo, hi), whole[lo:hi]), (lo, hi)
+    for members in (on[large], on[_lib.TILE_128X128]):
+        whole = run(0, members)
+        for lo in (0, members // 2, members - few):
+            assert torch.equal(run(lo, lo + few), whole[lo:lo + few]), (members, lo)
+
+
+@pytest.mark.parametrize('dout', [384, 512])
+@pytest.mark.parametrize('din', [128, 192, 256, 320, 1536])
+def test_dense_depths_around_the_steady_loop_on_every_tile(din, dout):
+    """The dense product runs k stages 1 .. din / 32 - 4 from its steady loop in pairs: none at 4 or 6 stages, one pair at
+    8 and 10, 22 at 48, and each tile has its own number of loads in flight. The fewest rows that take each tile (the
+    large ones from a depth of 192 or 256 on), ragged in every tile: within one bf16 step of x W^T, and the same bits as
+    its last members on 64 x 64 tiles, from a WTILE weight, and from TILE16 rows."""
+    from tests._util import tile16_index
+    T = 240
+    on = _members_on_tiles(T, din, dout, _lib.RESULT_BF16)
+    large = _lib.TILE_256X128 if dout % 256 else _lib.TILE_256X256
+    assert {_lib.TILE_128X128, _lib.TILE_64X64} <= set(on) and (large in on or din < (256 if dout % 256 else 192))
+    g = torch.Generator(DEV).manual_seed(48)
+    w = (torch.randn(dout, din, device=DEV, generator=g) * din ** -0.5).bfloat16()
+    wt = torch.empty_like(w)
+    _lib.call('noise_weight_tiles', w.data_ptr(), dout, din, wt.data_ptr(), _stream())
+
+    def run(x, members, x_layout=_lib.LAYOUT_ROWS, weight=w, w_layout=_lib.LAYOUT_ROWS):
+        y = torch.empty(members * T, dout, device=DEV, dtype=torch.bfloat16)
+        _lib.call('noise_dense_bf16', x.data_ptr(), x_layout, din, dout, weight.data_ptr(), w_layout, members, T,
+                  y.data_ptr(), _stream())
+        torch.cuda.synchronize()
+        return y
+    for tile, members in on.items():
+        log_case(f'dense depth {din}->{dout} on tile {tile}: {members} members of {T} rows')
+        x = torch.randn(members * T, din, device=DEV, generator=g).bfloat16()
+        y = run(x, members)
+        ref = (x.float() @ w.float().t()).bfloat16().float()
+        assert ((y.float() - ref).abs() <= ref.abs() * 2 ** -7 + 1e-6).all()
+        assert torch.equal(run(x[-3 * T:], min(3, members)), y[-3 * T:])
+        with torch.device(DEV):
+            at = tile16_index(members * T, din).flatten()
+        x16 = torch.empty_like(x)
+        x16.view(-1)[at] = x.view(-1)
+        assert torch.equal(run(x, members, weight=wt, w_layout=_lib.LAYOUT_WTILE), y)
+        assert torch.equal(run(x16, members, _lib.LAYOUT_TILE16, wt, _lib.LAYOUT_WTILE), y)
 
 
 @pytest.mark.parametrize('T', [256, 250])
 @pytest.mark.parametrize('head', ['fp32', 'bf16', 'fp32_split'])
 def test_tile_configurations_of_the_head_agree_bit_for_bit(head, T):
-    """The same for the head's per-token losses: 16,384 rows (256 x 256 tiles), 2,560 (128 x 128) and one member
-    (64 x 64), from tiled operands (T = 256) and row-major ones with straddling tiles (T = 250)."""
+    """The same for the head's per-token losses: the fewest rows that take each of its three tiles, against members at
+    either end and in the middle on 64 x 64 tiles, from tiled operands (T = 256) and row-major ones with straddling tiles
+    (T = 250)."""
     from noise_amd.population import HEAD_FORMAT
     g = torch.Generator().manual_seed(33)
-    P, V, fmt = 64, 4096, HEAD_FORMAT[head]
-    log_case(f'head tile configurations {head} T={T}')
+    V, fmt = 4096, HEAD_FORMAT[head]
+    on = _members_on_tiles(T, {'bf16': 512, 'fp32': 1024, 'fp32_split': 1536}[head], V, _lib.RESULT_HEAD, 40000)
+    assert set(on) == {_lib.TILE_256X256, _lib.TILE_128X128, _lib.TILE_64X64} and on[_lib.TILE_64X64] == 1
+    P = max(on.values())
+    log_case(f'head tile configurations {head} T={T}: members {on}')
     x = torch.randn(P * T, 512, generator=g).to(DEV)
     w = (torch.randn(V, 512, generator=g) * 0.05).to(DEV)
     op = w
@@ -99,9 +156,10 @@ def test_tile_configurations_of_the_head_agree_bit_for_bit(head, T):
                   None, ws.data_ptr(), n, None, 0, _stream())
         torch.cuda.synchronize()
         return loss
-    whole = run(0, P)
-    for lo, hi in ((4, 14), (P - 1, P)):
-        assert torch.equal(run(lo, hi), whole[lo * T:hi * T]), (lo, hi)
+    for members in (on[_lib.TILE_256X256], on[_lib.TILE_128X128]):
+        whole = run(0, members)
+        for lo in (0, members // 2, members - 1):
+            assert torch.equal(run(lo, lo + 1), whole[lo * T:(lo + 1) * T]), (members, lo)
 
 
 @pytest.mark.parametrize('shared', ['q', 'k'])
