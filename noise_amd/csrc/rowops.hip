@@ -642,11 +642,14 @@ int block_entry_launch(const BlockEntryArgs& g, hipStream_t s) {
   if (g.gate_w && (!g.gate_a || !g.gate_b || !g.gate || (((uintptr_t)g.gate_w | (uintptr_t)g.gate_b) & 15)))
     return NOISE_EINVAL;
   if (bad_pending(g.pend, g.npend)) return NOISE_EINVAL;
-  // a wave per row up to 32 rows per CU: a workgroup of 8 rows then holds its CU alone for two row latencies and the
-  // staging of its vectors (256 rows 7.8 -> 5.0 us, 2048 9.0 -> 6.5, 8192 15.2 -> 14.3; at 32,768 block 0 loses, 30.9 ->
-  // 34.4)
+  // a wave per row in launches of few rows: a workgroup of 8 rows then holds its CU alone for two row latencies and the
+  // staging of its vectors (256 rows 7.8 -> 5.0 us, 2048 9.0 -> 6.5, 8192 of one member 15.2 -> 14.3; at 32,768 block 0
+  // loses, 30.9 -> 34.4). Up to 32 rows per CU; behind deferred residuals, whose four more vectors each row then reads by
+  // itself, only where members of 256 rows or more share them, and 16 otherwise (8192 rows of 128, 64, 32 and 8 per member
+  // 13.1, 13.0, 13.3 and 15.0 us by groups, 13.6, 14.7, 16.5 and 17.3 by rows; 4096 rows of 8 8.8 and 8.3).
   const bool first = !g.x_in && !g.x0 && !g.npend;
-  const bool grouped = g.T % GROUP_ROWS == 0 && g.M % GROUP_ROWS == 0 && g.M > 32 * num_cus();
+  const bool grouped = g.T % GROUP_ROWS == 0 && g.M % GROUP_ROWS == 0 &&
+                       g.M > (first || g.T >= 256 ? 32 : 16) * num_cus();
   if (first && grouped)
     hipLaunchKernelGGL(block_entry_group_kernel<true>, dim3((unsigned)(g.M / GROUP_ROWS)), dim3(256), 0, s, g);
   else if (first)
