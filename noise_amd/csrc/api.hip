@@ -1,4 +1,5 @@
 // extern "C" entry points of libnoise_hip.so (declared in include/noise_hip.h).
+#include <algorithm>
 #include <mutex>
 #include <vector>
 
@@ -214,13 +215,22 @@ int noise_cast_bf16(const float* in, void* out, long n, int split_cols, noise_st
 
 int noise_cast_weights(const noise_cast_t* mats, int n, noise_stream_t stream) {
   if (n <= 0 || !mats) return NOISE_EINVAL;
-  std::vector<CastMat> m(n);
+  const auto mat = [&](int k) {
+    const noise_cast_t& c = mats[k];
+    return CastMat{c.in, static_cast<bf16*>(c.out), (long)c.rows * c.cols, c.cols, c.layout == NOISE_LAYOUT_WTILE};
+  };
+  // every matrix is checked before the first launch: a rejected call writes nothing
   for (int k = 0; k < n; ++k) {
     if (mats[k].layout != NOISE_LAYOUT_ROWS && mats[k].layout != NOISE_LAYOUT_WTILE) return NOISE_EINVAL;
-    m[k] = CastMat{mats[k].in, static_cast<bf16*>(mats[k].out), (long)mats[k].rows * mats[k].cols, mats[k].cols,
-                   mats[k].layout == NOISE_LAYOUT_WTILE};
+    if (int rc = cast_check(mat(k))) return rc;
   }
-  return cast_batch_launch(m.data(), n, static_cast<hipStream_t>(stream));
+  for (int base = 0; base < n; base += CAST_MAX) {
+    CastBatchArgs g{};
+    g.n = std::min(CAST_MAX, n - base);
+    for (int k = 0; k < g.n; ++k) g.m[k] = mat(base + k);
+    if (int rc = cast_batch_launch(g, static_cast<hipStream_t>(stream))) return rc;
+  }
+  return NOISE_OK;
 }
 
 int noise_embed_norm(const float* w, long vocab, const float* a, const float* b, const float* sign,

@@ -133,4 +133,5 @@ struct CastBatchArgs {
   CastMat m[CAST_MAX];
   int n;
 };
-int cast_batch_launch(const CastMat* mats, int n, hipStream_t s);
+int cast_check(const CastMat& m);
+int cast_batch_launch(CastBatchArgs& g, hipStream_t s);  // g.m[0 .. g.n): checked matrices

@@ -713,28 +713,22 @@ int token_range_launch(const int64_t* a, long na, const int64_t* b, long nb, int
   return NOISE_OK;
 }
 
-int cast_batch_launch(const CastMat* mats, int n, hipStream_t s) {
-  if (n <= 0 || !mats) return NOISE_EINVAL;
-  // every matrix is checked before the first launch: a rejected call writes nothing
-  for (int k = 0; k < n; ++k) {
-    const CastMat& m = mats[k];
-    if (!m.in || !m.out || m.n <= 0 || m.cols <= 0 || m.n % m.cols ||
-        (m.tiled && (m.cols % 32 || m.n / m.cols % 64 || ((uintptr_t)m.out & 15))))
-      return NOISE_EINVAL;
-    if (m.n > (long)CAST_BLOCK * (0x7fffffff / CAST_MAX)) return NOISE_ENOTSUP;
+int cast_check(const CastMat& m) {
+  if (!m.in || !m.out || m.n <= 0 || m.cols <= 0 || m.n % m.cols ||
+      (m.tiled && (m.cols % 32 || m.n / m.cols % 64 || ((uintptr_t)m.out & 15))))
+    return NOISE_EINVAL;
+  return m.n > (long)CAST_BLOCK * (0x7fffffff / CAST_MAX) ? NOISE_ENOTSUP : NOISE_OK;
+}
+
+int cast_batch_launch(CastBatchArgs& g, hipStream_t s) {
+  int blocks = 0;
+  for (int k = 0; k < g.n; ++k) {
+    CastMat& m = g.m[k];
+    m.vec = !(((uintptr_t)m.in | (uintptr_t)m.out) & 15);
+    blocks += (int)((m.n + CAST_BLOCK - 1) / CAST_BLOCK);
+    m.block_end = blocks;
   }
-  for (int base = 0; base < n; base += CAST_MAX) {
-    CastBatchArgs g{};
-    g.n = n - base < CAST_MAX ? n - base : CAST_MAX;
-    int blocks = 0;
-    for (int k = 0; k < g.n; ++k) {
-      CastMat& m = g.m[k] = mats[base + k];
-      m.vec = !(((uintptr_t)m.in | (uintptr_t)m.out) & 15);
-      blocks += (int)((m.n + CAST_BLOCK - 1) / CAST_BLOCK);
-      m.block_end = blocks;
-    }
-    hipLaunchKernelGGL(cast_batch_kernel, dim3((unsigned)blocks), dim3(256), 0, s, g);
-    NOISE_CHECK_LAUNCH();
-  }
+  hipLaunchKernelGGL(cast_batch_kernel, dim3((unsigned)blocks), dim3(256), 0, s, g);
+  NOISE_CHECK_LAUNCH();
   return NOISE_OK;
 }

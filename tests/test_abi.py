@@ -84,6 +84,12 @@ def test_bad_arguments_are_rejected_without_touching_the_gpu():
     assert lib.noise_adam_batch(ptr, count, .5, .95, 1e-8, None) == EINVAL
     ptr, count, _keep = _lib.adam_tensors([good] * 70 + [(16, 16, 16, 16, 256, 1e-3, 0.0)])  # bc2_sqrt must be > 0
     assert lib.noise_adam_batch(ptr, count, .5, .95, 1e-8, None) == EINVAL
+    # casts: a matrix past the first launch refuses the call before any launch, and a rejected call takes no memory by
+    # the count it names (a host array of that many would not fit)
+    ptr, count, _keep = _lib.casts([(16, 16, 64, 32, _lib.LAYOUT_ROWS)] * 70 + [(16, 16, 63, 32, _lib.LAYOUT_WTILE)])
+    assert lib.noise_cast_weights(ptr, count, None) == EINVAL
+    ptr, _count, _keep = _lib.casts([(16, 16, 64, 32, 7)])
+    assert lib.noise_cast_weights(ptr, 0x7fffffff, None) == EINVAL
     assert lib.noise_attention(1, 1, 100, 50, 0, 1, None, 0, 1, None, None, None, 0, None) == EINVAL  # T % 128
     # bf16 q, k, v with bf16 probabilities exists only for RMS-normalised q, k (the bounded-score softmax)
     assert lib.noise_attention(16, 1, 128, 50, 0, 3, None, 0, 16, None, None, None, 0, None) == EINVAL
