@@ -331,7 +331,7 @@ def run_head(args):
                     'head': HEAD_DESC[args.head], 'sigma': SIGMA, 'gpus': 1},
                    {'bound': 'mfma', 'achieved': achieved, 'peak': PEAK_BF16_TFLOPS, 'unit': 'TFLOP/s',
                     'frac': achieved / PEAK_BF16_TFLOPS, 'traffic': None,
-                    'kernel': 'head_norm + lowrank_gemm<EPI_CE%s> + ce_finalize' % ('_F16' if fmt == _lib.HEAD_FP32 else ''),
+                    'kernel': 'head_norm + lowrank_gemm<EPI_CE%s> + ce_rows' % ('_F16' if fmt == _lib.HEAD_FP32 else ''),
                     'flop_per_launch': flop,
                     'ms_per_launch': ms_launch})
 

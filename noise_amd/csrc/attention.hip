@@ -82,8 +82,8 @@ __device__ __forceinline__ int vsw(int R) { return 2 * (((R >> 1) & 1) | ((((R >
 
 // Edge-block masks as lane masks. A lane (query row r = lane % 16, lane group g = lane / 16) holds, for MFMA key block
 // kb and element e, the key kstart + 8 g + ko with ko = 32 (kb / 2) + 4 (kb % 2) + e. Against its query
-// q0 + 32 wave + 16 qb + r the causal test key <= q reads v >= t with v = r - 8 g (a per-lane constant, -24 .. 15) and
-// t = ko + t0, t0 = kstart - q0 - 32 wave - 16 qb (uniform); the window test key >= q - window reads the complement
+// q0 + 16 QB wave + 16 qb + r the causal test key <= q reads v >= t with v = r - 8 g (a per-lane constant, -24 .. 15) and
+// t = ko + t0, t0 = kstart - q0 - 16 QB wave - 16 qb (uniform); the window test key >= q - window reads the complement
 // v < t + window + 1. The set of lanes with v >= t depends on t alone: LANES_GE[t + 64] holds it as a 64-bit lane
 // mask for t in [-64, 80) (all lanes below -24, none above 15), so a block's 16 masks per query block come from two
 // scalar loads of 8 consecutive entries (ko = 0..7 and 32..39, t0 clamped to [-64, 40] where the masks saturate) and
@@ -161,7 +161,7 @@ __global__ void __launch_bounds__(NTH, 4) attention_kernel(AttnArgs g) {
   };
   const bf16 *qh = heads(g.q), *kh = heads(g.k), *vh = heads(g.v);
 
-  // Q fragments (MFMA B operand): query q0 + 32 wave + 16 qb + lane % 16, dims 32 kk + 8 grp ..
+  // Q fragments (MFMA B operand): query q0 + 16 QB wave + 16 qb + lane % 16, dims 32 kk + 8 grp ..
   bf16x8 qf[QB][2];
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb)
